@@ -1,9 +1,8 @@
 // csr_kernels.hip — CSR family on 64-lane wavefronts (gfx950).
 //
 //   CSR_DIRECT         a lane group of G lanes owns one row; each lane keeps V
-//                      packets (float4 when N % 4 == 0 and buffers are 16-byte
-//                      aligned, float otherwise) of the output row, so one
-//                      wave-wide dwordx4 load gathers 64/G whole B rows.
+//                      packets (4 columns; 1 where N < 4) of the output row, so
+//                      one wave-wide dwordx4 load gathers 64/G whole B rows.
 //                      (col, val) of a G-wide slice of the row are loaded
 //                      coalesced, one per lane, and broadcast with ds_bpermute.
 //   baseline           regime-free reference point: one wave per row, lanes
@@ -25,6 +24,7 @@
 #include <cstdlib>
 #include <chrono>
 #include <mutex>
+#include <type_traits>
 
 #include "ra_internal.hpp"
 #include "zo_plan.hpp"
@@ -43,111 +43,193 @@ using ra::kChunk;
 using ra::kSoleFlag;
 
 // ------------------------------------------------------------------ packets
+// A packet is the run of output columns one lane owns: 4 floats, or 1 where
+// N < 4.  A 4-float packet needs 4-byte alignment only (a dwordx4 access on
+// gfx950 does), so any N >= 4 and any float buffer takes 16-byte accesses: the
+// row's last packet starts at N - 4, is loaded whole and stores only the
+// columns no other packet owns (own_from).  With 4-byte packets a row of N = 47
+// took a whole wave: a power-law graph of 1e6 rows and 2.6e7 nonzeros ran 1.07
+// ms at N = 47, now 0.97 ms, one of 2e5 rows 57.9 us at N = 31, now 46.5 us.
+// What is left over N = 48 (0.80 ms) is the unaligned rows' extra 64-byte
+// sectors.
+typedef float pk4 __attribute__((ext_vector_type(4), aligned(4)));
+
 template <typename P> __device__ __forceinline__ P pzero();
 template <> __device__ __forceinline__ float pzero<float>() { return 0.f; }
-template <> __device__ __forceinline__ float4 pzero<float4>() { return make_float4(0.f, 0.f, 0.f, 0.f); }
+template <> __device__ __forceinline__ pk4 pzero<pk4>() { return pk4{0.f, 0.f, 0.f, 0.f}; }
 
 __device__ __forceinline__ float pfma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ __forceinline__ float4 pfma(float a, float4 b, float4 c) {
-    return make_float4(__builtin_fmaf(a, b.x, c.x), __builtin_fmaf(a, b.y, c.y),
-                       __builtin_fmaf(a, b.z, c.z), __builtin_fmaf(a, b.w, c.w));
+__device__ __forceinline__ pk4 pfma(float a, pk4 b, pk4 c) {
+    return pk4{__builtin_fmaf(a, b.x, c.x), __builtin_fmaf(a, b.y, c.y), __builtin_fmaf(a, b.z, c.z),
+               __builtin_fmaf(a, b.w, c.w)};
 }
 __device__ __forceinline__ float padd(float a, float b) { return a + b; }
-__device__ __forceinline__ float4 padd(float4 a, float4 b) {
-    return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+__device__ __forceinline__ pk4 padd(pk4 a, pk4 b) { return pk4{a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w}; }
+
+template <typename P> struct PacketElems;
+template <> struct PacketElems<float> { static constexpr int value = 1; };
+template <> struct PacketElems<pk4> { static constexpr int value = 4; };
+
+// First column of packet qq of an N-column row.  Lanes past the row's end
+// repeat its last packet (the same address, so no extra traffic) and store
+// nothing.
+template <typename P>
+__device__ __forceinline__ int packet_column(int qq, int N) {
+    constexpr int E = PacketElems<P>::value;
+    return min(qq * E, N - E);
 }
 
 // Streaming (non-temporal) accesses for data touched once: the CSR index and
 // value streams and the C rows.  They then do not displace B rows that other
 // waves are about to gather again from L2.
-typedef float f32x4n __attribute__((ext_vector_type(4)));
 template <typename T>
 __device__ __forceinline__ T load_once(const T* p, bool nt) {
     return nt ? __builtin_nontemporal_load(p) : *p;
 }
-__device__ __forceinline__ void store_once(float* p, float v, bool nt) {
-    if (nt) __builtin_nontemporal_store(v, p);
-    else *p = v;
+// The empty asm keeps the two stores apart: merged into one instruction they
+// lose the hint.
+template <typename P>
+__device__ __forceinline__ void store_once(float* p, P v, bool nt) {
+    if (nt) {
+        asm volatile("" ::: "memory");
+        __builtin_nontemporal_store(v, reinterpret_cast<P*>(p));
+        asm volatile("" ::: "memory");
+    } else {
+        *reinterpret_cast<P*>(p) = v;
+    }
 }
-__device__ __forceinline__ void store_once(float4* p, float4 v, bool nt) {
-    if (nt) __builtin_nontemporal_store(f32x4n{v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4n*>(p));
-    else *p = v;
+
+template <typename P>
+__device__ __forceinline__ P load_packet(const float* row, int col) {
+    return *reinterpret_cast<const P*>(row + col);
+}
+
+// Where the gathered B rows are.  A row's key is what the lanes of a group hand
+// each other; a nonzero past the end of a row has the key kNone and gathers 0.
+//
+// BufferRows: key = byte offset of the row, gathered through a buffer
+// descriptor whose bounds check returns 0 for kNone, so a round of gathers is
+// U loads back to back with no branch or mask between them (with a branch per
+// gather the compiler waits for earlier loads in between).  Where the chain of
+// one long row sets the time this is most of it: a power-law graph of 20,000
+// rows at N = 64 went from 44 to 25 us, one of 1e6 rows at N = 16 from 280 to
+// 244 us; at N = 128 and 256, bound by the gathered bytes, nothing changed.
+// Offsets are 32 bits: B up to kBufferLimit bytes, rows up to kBufferRow
+// columns.  PointerRows: 64-bit addresses, for anything larger.
+constexpr uint32_t kBufferLimit = 0xFFFF0000u;
+constexpr int kBufferRow = 16000;  // kNone + a column's byte offset stays below 2^32
+
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+struct BufferRows {
+    typedef uint32_t Key;
+    static constexpr Key kNone = kBufferLimit;
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t row_bytes;
+    __device__ __forceinline__ BufferRows(const float* B, int N)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(B), 0, static_cast<int>(kBufferLimit), 0x00027000)),
+          row_bytes(N * 4u) {}
+    __device__ __forceinline__ Key key(int col) const { return static_cast<uint32_t>(col) * row_bytes; }
+    template <typename P>
+    __device__ __forceinline__ P load(Key k, int col) const {
+        if constexpr (PacketElems<P>::value == 4)
+            return __builtin_bit_cast(P, __builtin_amdgcn_raw_buffer_load_b128(rsrc, k + col * 4u, 0, 0));
+        else
+            return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, k + col * 4u, 0, 0));
+    }
+};
+
+struct PointerRows {
+    typedef int Key;
+    static constexpr Key kNone = -1;
+    const float* B;
+    int64_t ld;
+    __device__ __forceinline__ PointerRows(const float* b, int N) : B(b), ld(N) {}
+    __device__ __forceinline__ Key key(int col) const { return col; }
+    template <typename P>
+    __device__ __forceinline__ P load(Key k, int col) const {
+        return k >= 0 ? load_packet<P>(B + k * ld, col) : pzero<P>();
+    }
+};
+
+// Store packet qq (whose first column is col) into an N-column row.
+__device__ __forceinline__ void store_packet(float* row, int qq, int col, float v, bool nt) {
+    if (qq == col) store_once(row + col, v, nt);
+}
+__device__ __forceinline__ void store_packet(float* row, int qq, int col, pk4 v, bool nt) {
+    const int own_from = 4 * qq - col;  // 1..3: last packet of a ragged row; >= 4: past the row's end
+    if (own_from == 0) {
+        store_once(row + col, v, nt);
+        return;
+    }
+    if (own_from < 4) store_once(row + col + 3, v.w, nt);
+    if (own_from < 3) store_once(row + col + 2, v.z, nt);
+    if (own_from < 2) store_once(row + col + 1, v.y, nt);
+}
+
+// One round: U gathered packets per lane and their fmas, in order.  A key of
+// kNone comes with the value -0: adding 0 * -0 = -0 changes no accumulator, the
+// sign of a zero included.
+template <int V, int U, typename P, typename Rows>
+__device__ __forceinline__ void gather_round(const Rows& rows, const typename Rows::Key (&c)[U], const float (&a)[U],
+                                             const int (&q)[V], P (&acc)[V]) {
+    P b[U][V];
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+#pragma unroll
+        for (int s = 0; s < V; ++s) b[k][s] = rows.template load<P>(c[k], q[s]);
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+#pragma unroll
+        for (int s = 0; s < V; ++s) acc[s] = pfma(a[k], b[k][s], acc[s]);
 }
 
 // Accumulate the nnz range [p0, p1) of one row into acc.  All G lanes of the
-// group share the range; lane `sl` owns packet columns q[s] (q < 0: masked).
+// group share the range; lane `sl` gathers the packets at columns q[s].
 // Per output element the update order is p ascending, one fma per nonzero.
-template <int G, int V, int U, typename P>
+template <int G, int V, int U, typename P, typename Rows>
 __device__ __forceinline__ void accumulate_range(const int32_t* __restrict__ colind,
-                                                 const float* __restrict__ vals,
-                                                 const P* __restrict__ Bp, int64_t ldp,
+                                                 const float* __restrict__ vals, const Rows& rows,
                                                  int p0, int p1, int sl, const int (&q)[V],
                                                  P (&acc)[V], bool nt) {
     static_assert(U <= G, "unroll deeper than the lane group");
     for (int base = p0; base < p1; base += G) {
         const int my = base + sl;
-        int mc = 0;
-        float mv = 0.f;
+        typename Rows::Key mc = Rows::kNone;
+        float mv = -0.f;
         if (my < p1) {
-            mc = load_once(colind + my, nt);
+            mc = rows.key(load_once(colind + my, nt));
             mv = load_once(vals + my, nt);
         }
         const int cnt = min(G, p1 - base);
         for (int j = 0; j < cnt; j += U) {
-            int c[U];
+            typename Rows::Key c[U];
             float a[U];
 #pragma unroll
             for (int k = 0; k < U; ++k) {
                 c[k] = __shfl(mc, j + k, G);
                 a[k] = __shfl(mv, j + k, G);
             }
-            P b[U][V];
-#pragma unroll
-            for (int k = 0; k < U; ++k) {
-#pragma unroll
-                for (int s = 0; s < V; ++s) {
-                    b[k][s] = (j + k < cnt && q[s] >= 0) ? Bp[(int64_t)c[k] * ldp + q[s]]
-                                                        : pzero<P>();
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < U; ++k) {
-                if (j + k < cnt) {
-#pragma unroll
-                    for (int s = 0; s < V; ++s) acc[s] = pfma(a[k], b[k][s], acc[s]);
-                }
-            }
+            gather_round<V, U, P>(rows, c, a, q, acc);
         }
     }
 }
 
-// As accumulate_range, with the (column, value) pairs of [p0, p1) already in
-// LDS (s_col / s_val indexed from the chunk start): one broadcast LDS read per
+// As accumulate_range over entries [p0, p1) of a chunk whose (key, value) pairs
+// are in LDS, (kNone, -0) from the chunk's end on: one broadcast LDS read per
 // pair instead of a coalesced global load and a lane shuffle.
-template <int G, int V, int U, typename P>
-__device__ __forceinline__ void accumulate_lds(const int32_t* s_col, const float* s_val,
-                                               const P* __restrict__ Bp, int64_t ldp, int p0, int p1,
-                                               const int (&q)[V], P (&acc)[V]) {
+template <int V, int U, typename P, typename Rows>
+__device__ __forceinline__ void accumulate_lds(const typename Rows::Key* s_key, const float* s_val, const Rows& rows,
+                                               int p0, int p1, const int (&q)[V], P (&acc)[V]) {
     for (int p = p0; p < p1; p += U) {
-        int c[U];
+        typename Rows::Key c[U];
         float a[U];
 #pragma unroll
         for (int k = 0; k < U; ++k) {
-            c[k] = p + k < p1 ? s_col[p + k] : 0;
-            a[k] = p + k < p1 ? s_val[p + k] : 0.f;
+            c[k] = s_key[p + k];
+            a[k] = s_val[p + k];
         }
-        P b[U][V];
-#pragma unroll
-        for (int k = 0; k < U; ++k)
-#pragma unroll
-            for (int s = 0; s < V; ++s)
-                b[k][s] = (p + k < p1 && q[s] >= 0) ? Bp[(int64_t)c[k] * ldp + q[s]] : pzero<P>();
-#pragma unroll
-        for (int k = 0; k < U; ++k)
-            if (p + k < p1) {
-#pragma unroll
-                for (int s = 0; s < V; ++s) acc[s] = pfma(a[k], b[k][s], acc[s]);
-            }
+        gather_round<V, U, P>(rows, c, a, q, acc);
     }
 }
 
@@ -177,12 +259,11 @@ __device__ __forceinline__ int64_t block_and_slice(bool remap, int nslices, int&
 }
 
 // ---------------------------------------------------------------- CSR_DIRECT
-template <int G, int V, int U, typename P>
+template <int G, int V, int U, typename P, typename Rows>
 __global__ __launch_bounds__(kBlock) void csr_rows_kernel(
     const int32_t* __restrict__ rowptr, const int32_t* __restrict__ colind,
-    const float* __restrict__ vals, const P* __restrict__ Bp, P* __restrict__ Cp,
-    const int32_t* __restrict__ row_list, int64_t num_rows, int64_t ldp, int np, int remap,
-    int nt, int resume, int nslices) {
+    const float* __restrict__ vals, const float* __restrict__ B, float* __restrict__ C,
+    int64_t num_rows, int N, int remap, int nt, int resume, int nslices) {
     constexpr int RPW = kWave / G;
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
@@ -191,25 +272,24 @@ __global__ __launch_bounds__(kBlock) void csr_rows_kernel(
     int slice;
     const int64_t idx = (block_and_slice(remap, nslices, slice) * kWavesPerBlock + wave) * RPW + sub;
     if (idx >= num_rows) return;  // whole lane groups leave together
-    const int row = row_list ? row_list[idx] : static_cast<int>(idx);
-    const int q0 = slice * (G * V);
+    const int row = static_cast<int>(idx);
+    const int64_t ld = N;
+    const int q0 = slice * (G * V) + sl;
     int q[V];
 #pragma unroll
-    for (int s = 0; s < V; ++s) {
-        const int qq = q0 + sl + s * G;
-        q[s] = qq < np ? qq : -1;
-    }
+    for (int s = 0; s < V; ++s) q[s] = packet_column<P>(q0 + s * G, N);
+    float* crow = C + (int64_t)row * ld;
     // resume: the fma chain continues from C (a later column range of the same
     // rows; storing and reloading the fp32 accumulator changes no bit).
     P acc[V];
 #pragma unroll
     for (int s = 0; s < V; ++s)
-        acc[s] = (resume && q[s] >= 0) ? Cp[(int64_t)row * ldp + q[s]] : pzero<P>();
-    accumulate_range<G, V, U, P>(colind, vals, Bp, ldp, rowptr[row], rowptr[row + 1], sl, q, acc,
-                                 nt != 0);
+        acc[s] = resume ? load_packet<P>(crow, q[s]) : pzero<P>();
+    const Rows rows(B, N);
+    accumulate_range<G, V, U, P>(colind, vals, rows, rowptr[row], rowptr[row + 1], sl, q, acc, nt != 0);
 #pragma unroll
     for (int s = 0; s < V; ++s)
-        if (q[s] >= 0) store_once(Cp + (int64_t)row * ldp + q[s], acc[s], nt != 0);
+        store_packet(crow, q0 + s * G, q[s], acc[s], nt != 0);
 }
 
 // ----------------------------------------------------------------- baseline
@@ -251,17 +331,16 @@ __global__ __launch_bounds__(kBlock) void csr_baseline_kernel(
 // contiguous parts that are summed in group order through LDS (with
 // RA_ZO_SOLE_SPLIT=1 sole chunks are split the same way; measured no faster
 // on C2 and C5).  Later waves take 64/G rows of the short-row list each.
-template <int G, int V, int U, typename P>
+template <int G, int V, int U, typename P, typename Rows>
 __global__ __launch_bounds__(kBlock) void zo_fused_kernel(
     const int32_t* __restrict__ rowptr, const int32_t* __restrict__ colind,
-    const float* __restrict__ vals, const P* __restrict__ Bp, P* __restrict__ Cp,
+    const float* __restrict__ vals, const float* __restrict__ B, float* __restrict__ C,
     const int32_t* __restrict__ chunk_rows, const int32_t* __restrict__ chunk_starts,
-    const int32_t* __restrict__ chunk_slot, int num_chunks, P* __restrict__ partials,
-    const int32_t* __restrict__ short_rows, int64_t num_short, int64_t ldp, int np, int remap,
-    int nt, int sole_split, int nslices, int lds_stage) {
+    const int32_t* __restrict__ chunk_slot, int num_chunks, float* __restrict__ partials,
+    const int32_t* __restrict__ short_rows, int64_t num_short, int N, int remap, int nt, int sole_split, int nslices, int lds_stage) {
     constexpr int RPW = kWave / G;
     __shared__ P red[kWavesPerBlock][(RPW > 1 ? RPW - 1 : 1) * G * V];
-    __shared__ int s_col[kWavesPerBlock][kChunk];
+    __shared__ typename Rows::Key s_key[kWavesPerBlock][kChunk];
     __shared__ float s_val[kWavesPerBlock][kChunk];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
@@ -269,16 +348,15 @@ __global__ __launch_bounds__(kBlock) void zo_fused_kernel(
     const int sl = lane % G;
     int slice;
     const int64_t gw = block_and_slice(remap, nslices, slice) * kWavesPerBlock + wave;
-    const int q0 = slice * (G * V);
+    const int64_t ld = N;
+    const int q0 = slice * (G * V) + sl;
     int q[V];
 #pragma unroll
-    for (int s = 0; s < V; ++s) {
-        const int qq = q0 + sl + s * G;
-        q[s] = qq < np ? qq : -1;
-    }
+    for (int s = 0; s < V; ++s) q[s] = packet_column<P>(q0 + s * G, N);
     P acc[V];
 #pragma unroll
     for (int s = 0; s < V; ++s) acc[s] = pzero<P>();
+    const Rows rows(B, N);
 
     if (gw < num_chunks) {
         const uint32_t tag = static_cast<uint32_t>(chunk_rows[gw]);
@@ -289,9 +367,16 @@ __global__ __launch_bounds__(kBlock) void zo_fused_kernel(
             // The chunk's (column, value) pairs go to LDS first, in one
             // coalesced pass by the whole wave (RA_ZO_LDS_STAGE=0: loaded G at a
             // time and shuffled, as for the short rows).
-            for (int i = lane; i < ce - cs; i += kWave) {
-                s_col[wave][i] = load_once(colind + cs + i, nt != 0);
-                s_val[wave][i] = load_once(vals + cs + i, nt != 0);
+#pragma unroll
+            for (int i = lane; i < kChunk; i += kWave) {
+                typename Rows::Key key = Rows::kNone;
+                float val = -0.f;
+                if (i < ce - cs) {
+                    key = rows.key(load_once(colind + cs + i, nt != 0));
+                    val = load_once(vals + cs + i, nt != 0);
+                }
+                s_key[wave][i] = key;
+                s_val[wave][i] = val;
             }
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
             __builtin_amdgcn_wave_barrier();
@@ -301,18 +386,18 @@ __global__ __launch_bounds__(kBlock) void zo_fused_kernel(
             // single fma chain per element, as for the short rows: the same
             // bits as CSR_DIRECT (csr/ra_zero_overhead.cu:246-262).
             if (sub != 0) return;
-            if (lds_stage) accumulate_lds<G, V, U, P>(s_col[wave], s_val[wave], Bp, ldp, 0, ce - cs, q, acc);
-            else accumulate_range<G, V, U, P>(colind, vals, Bp, ldp, cs, ce, sl, q, acc, nt != 0);
+            if (lds_stage) accumulate_lds<V, U, P>(s_key[wave], s_val[wave], rows, 0, ce - cs, q, acc);
+            else accumulate_range<G, V, U, P>(colind, vals, rows, cs, ce, sl, q, acc, nt != 0);
 #pragma unroll
             for (int s = 0; s < V; ++s)
-                if (q[s] >= 0) store_once(Cp + (int64_t)row * ldp + q[s], acc[s], nt != 0);
+                store_packet(C + (int64_t)row * ld, q0 + s * G, q[s], acc[s], nt != 0);
             return;
         }
         constexpr int L = kChunk / RPW;
         const int a = min(cs + sub * L, ce);
         const int b = min(a + L, ce);
-        if (lds_stage) accumulate_lds<G, V, U, P>(s_col[wave], s_val[wave], Bp, ldp, a - cs, b - cs, q, acc);
-        else accumulate_range<G, V, U, P>(colind, vals, Bp, ldp, a, b, sl, q, acc, nt != 0);
+        if (lds_stage) accumulate_lds<V, U, P>(s_key[wave], s_val[wave], rows, a - cs, b - cs, q, acc);
+        else accumulate_range<G, V, U, P>(colind, vals, rows, a, b, sl, q, acc, nt != 0);
         if constexpr (RPW > 1) {
             if (sub > 0) {
 #pragma unroll
@@ -332,21 +417,21 @@ __global__ __launch_bounds__(kBlock) void zo_fused_kernel(
         }
         if (sub == 0) {
             const int slot = chunk_slot[gw];
-            P* dst = (tag & kSoleFlag) ? Cp + (int64_t)row * ldp : partials + (int64_t)slot * ldp;
+            float* dst = (tag & kSoleFlag) ? C + (int64_t)row * ld : partials + (int64_t)slot * ld;
 #pragma unroll
             for (int s = 0; s < V; ++s)
-                if (q[s] >= 0) store_once(dst + q[s], acc[s], nt != 0);
+                store_packet(dst, q0 + s * G, q[s], acc[s], nt != 0);
         }
         return;
     }
     const int64_t idx = (gw - num_chunks) * RPW + sub;
     if (idx >= num_short) return;
     const int row = short_rows[idx];
-    accumulate_range<G, V, U, P>(colind, vals, Bp, ldp, rowptr[row], rowptr[row + 1], sl, q, acc,
+    accumulate_range<G, V, U, P>(colind, vals, rows, rowptr[row], rowptr[row + 1], sl, q, acc,
                                  nt != 0);
 #pragma unroll
     for (int s = 0; s < V; ++s)
-        if (q[s] >= 0) store_once(Cp + (int64_t)row * ldp + q[s], acc[s], nt != 0);
+        store_packet(C + (int64_t)row * ld, q0 + s * G, q[s], acc[s], nt != 0);
 }
 
 // Deterministic merge: C[row] = ((slot0 + slot1) + slot2) + ... per element.
@@ -357,24 +442,26 @@ __global__ __launch_bounds__(kBlock) void zo_fused_kernel(
 template <typename P>
 __global__ __launch_bounds__(kBlock) void zo_merge_kernel(
     const int32_t* __restrict__ split_rows, const int32_t* __restrict__ split_off,
-    const P* __restrict__ partials, P* __restrict__ Cp, int64_t ldp, int np, int nrows) {
+    const float* __restrict__ partials, float* __restrict__ C, int N, int np, int nrows) {
     constexpr int D = 16;
     const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const int64_t r = t / np;
     if (r >= nrows) return;
     const int qq = static_cast<int>(t - r * np);
+    const int col = packet_column<P>(qq, N);
+    const int64_t ld = N;
     const int o0 = split_off[r], o1 = split_off[r + 1];
-    P acc = partials[(int64_t)o0 * ldp + qq];
+    P acc = load_packet<P>(partials + o0 * ld, col);
     int o = o0 + 1;
     for (; o + D <= o1; o += D) {
         P x[D];
 #pragma unroll
-        for (int i = 0; i < D; ++i) x[i] = partials[(int64_t)(o + i) * ldp + qq];
+        for (int i = 0; i < D; ++i) x[i] = load_packet<P>(partials + (o + i) * ld, col);
 #pragma unroll
         for (int i = 0; i < D; ++i) acc = padd(acc, x[i]);
     }
-    for (; o < o1; ++o) acc = padd(acc, partials[(int64_t)o * ldp + qq]);
-    Cp[(int64_t)split_rows[r] * ldp + qq] = acc;
+    for (; o < o1; ++o) acc = padd(acc, load_packet<P>(partials + o * ld, col));
+    store_packet(C + split_rows[r] * ld, qq, col, acc, false);
 }
 
 // ------------------------------------------------------------------ features
@@ -535,7 +622,7 @@ struct LaneShape {
 };
 
 // Tuning knobs, read once per process: RA_CSR_LANES forces the lane-group
-// width (4..64), RA_CSR_UNROLL the gathers in flight per lane (4 or 8),
+// width (4..64), RA_CSR_UNROLL the gathers in flight per lane (4, 8 or 16),
 // RA_XCD_REMAP=0 turns the XCD-contiguous block order of CSR_DIRECT off
 // (RA_ZO_XCD_REMAP=1 turns it on for ZERO_OVERHEAD_CSR, where it piles the hub
 // chunks onto one XCD), RA_CSR_STREAMING=0 turns the non-temporal hints off,
@@ -546,7 +633,7 @@ struct LaneShape {
 // pairs; RA_CSR_SLICE=c sets CSR_DIRECT's XCD-dealt column slice (0 off;
 // default 128 columns at N >= 256 when the unsliced grid has < 2^16 waves).
 struct CsrTuning {
-    int lanes = 0, unroll = 4, remap = 1, zo_remap = 0, nt = 1, coltile = 0, sole_split = 0, xslice = 0,
+    int lanes = 0, unroll = 0, remap = 1, zo_remap = 0, nt = 1, coltile = 0, sole_split = 0, xslice = 0,
         zo_slice = -1, lds_stage = 1, csr_slice = -1;
     CsrTuning() {
         if (const char* e = std::getenv("RA_CSR_SLICE")) csr_slice = std::atoi(e);
@@ -556,7 +643,7 @@ struct CsrTuning {
         if (const char* e = std::getenv("RA_ZO_SOLE_SPLIT")) sole_split = std::atoi(e) != 0;
         if (const char* e = std::getenv("RA_CSR_COLTILE")) coltile = std::atoi(e);
         if (const char* e = std::getenv("RA_CSR_LANES")) lanes = std::atoi(e);
-        if (const char* e = std::getenv("RA_CSR_UNROLL")) unroll = std::atoi(e) >= 8 ? 8 : 4;
+        if (const char* e = std::getenv("RA_CSR_UNROLL")) unroll = std::atoi(e) >= 16 ? 16 : std::atoi(e) >= 8 ? 8 : 4;
         if (const char* e = std::getenv("RA_XCD_REMAP")) remap = std::atoi(e) != 0;
         if (const char* e = std::getenv("RA_ZO_XCD_REMAP")) zo_remap = std::atoi(e) != 0;
         if (const char* e = std::getenv("RA_CSR_STREAMING")) nt = std::atoi(e) != 0;
@@ -570,6 +657,7 @@ const CsrTuning& tuning() {
 // Lane-group shape from the number of packets per row (per column pass).
 LaneShape pick_shape(int np, int packet_elems, int slice_elems = 0) {
     const CsrTuning& t = tuning();
+    if (packet_elems == 1) return {4, 1, 4};  // N < 4
     if (slice_elems > 0) np = std::min(np, std::max(1, slice_elems / packet_elems));
     else if (t.coltile > 0) np = std::min(np, std::max(1, t.coltile / packet_elems));
     int G;
@@ -577,21 +665,41 @@ LaneShape pick_shape(int np, int packet_elems, int slice_elems = 0) {
     else G = np <= 4 ? 4 : np <= 8 ? 8 : np <= 16 ? 16 : np <= 32 ? 32 : 64;
     int V = (np + G - 1) / G;
     V = V <= 1 ? 1 : V <= 2 ? 2 : 4;
-    const int U = std::min(G, t.unroll);
-    return {G, V, U};
+    return {G, V, 4};
 }
+
+// Gathers in flight per lane for a launch of `waves` waves.  A launch that does
+// not fill the chip several times over is bound by the latency of its longest
+// row's chain, and deeper rounds shorten it: power-law graphs at N = 64 of
+// 20,000 rows (6e3 waves) 25 / 19 / 16 us and 1e5 rows (3e4 waves) 40 / 35 / 39
+// us at 4 / 8 / 16 gathers.  A larger one is bound by the gathered bytes and
+// wants the waves that the registers cost (44 / 68 / 116 VGPRs): 2e5 rows at N
+// = 128 (1e5 waves) 76 / 82 / 102 us, 1e6 rows 888 / 916 / 988 us.
+int gathers_in_flight(const LaneShape& sh, int64_t waves) {
+    if (sh.V > 1) return 4;
+    const int u = tuning().unroll > 0 ? tuning().unroll : waves < (1 << 13) ? 16 : waves < (1 << 16) ? 8 : 4;
+    return std::min(sh.G, u);
+}
+
+// C is written with streaming stores where its rows are whole aligned packets
+// (1e6 rows at N = 16: 249 -> 244 us, at N = 128: 894 -> 888 us).  Ragged rows
+// share 16-byte runs with their neighbours, which the cache should merge: N =
+// 31 streamed 52.8 us, cached 46.5 us; N = 47 992 and 974 us.
+inline bool whole_packets(const float* C, int N) { return N % 4 == 0 && ra::aligned16(C); }
+
+// B and its rows fit the 32-bit offsets of BufferRows.
+inline bool buffer_rows_fit(int64_t K, int N) { return N <= kBufferRow && K * N * 4 <= int64_t{kBufferLimit}; }
 
 // True when grid.x * grid.y work-groups of kBlock lanes fit one grid dimension.
 inline bool fold_fits(dim3 grid) {
     return static_cast<uint64_t>(grid.x) * grid.y * kBlock <= 0xFFFFFFFFull;
 }
 
-template <typename P>
+template <typename P, typename Rows>
 ra_status launch_csr_rows(const LaneShape& sh, dim3 grid, hipStream_t st, const int32_t* rowptr,
-                          const int32_t* colind, const float* vals, const P* B, P* C,
-                          const int32_t* row_list, int64_t num_rows, int64_t ldp, int np, int resume,
-                          bool xcd_slices) {
-    const int remap = tuning().remap, nt = tuning().nt;
+                          const int32_t* colind, const float* vals, const float* B, float* C,
+                          int64_t num_rows, int N, int resume, bool xcd_slices) {
+    const int remap = tuning().remap, nt = tuning().nt && whole_packets(C, N);
     int nslices = 0;
     // Folding the column slices into grid.x is legal only while the folded
     // grid stays below 2^32 work-items (grid.x * blockDim on AMD); beyond
@@ -602,35 +710,42 @@ ra_status launch_csr_rows(const LaneShape& sh, dim3 grid, hipStream_t st, const 
     }
 #define RA_ROWS_CASE(g, v, u)                                                               \
     if (sh.G == g && sh.V == v && sh.U == u) {                                              \
-        csr_rows_kernel<g, v, u, P><<<grid, kBlock, 0, st>>>(rowptr, colind, vals, B, C,    \
-                                                             row_list, num_rows, ldp, np,   \
-                                                             remap, nt, resume, nslices);   \
+        csr_rows_kernel<g, v, u, P, Rows><<<grid, kBlock, 0, st>>>(                         \
+            rowptr, colind, vals, B, C, num_rows, N, remap, nt, resume, nslices);           \
         RA_LAUNCH_CHECK("csr_rows_kernel");                                                 \
         return RA_OK;                                                                       \
     }
 #define RA_ROWS_G(g, u) RA_ROWS_CASE(g, 1, u) RA_ROWS_CASE(g, 2, u) RA_ROWS_CASE(g, 4, u)
-    RA_ROWS_G(4, 4)
-    RA_ROWS_G(8, 4)
-    RA_ROWS_G(8, 8)
-    RA_ROWS_G(16, 4)
-    RA_ROWS_G(16, 8)
-    RA_ROWS_G(32, 4)
-    RA_ROWS_G(32, 8)
-    RA_ROWS_G(64, 4)
-    RA_ROWS_G(64, 8)
+    RA_ROWS_CASE(4, 1, 4)
+    if constexpr (PacketElems<P>::value == 4) {
+        RA_ROWS_CASE(4, 2, 4)
+        RA_ROWS_CASE(4, 4, 4)
+        RA_ROWS_G(8, 4)
+        RA_ROWS_G(16, 4)
+        RA_ROWS_G(32, 4)
+        RA_ROWS_G(64, 4)
+        if constexpr (std::is_same_v<Rows, BufferRows>) {
+            RA_ROWS_CASE(8, 1, 8)
+            RA_ROWS_CASE(16, 1, 8)
+            RA_ROWS_CASE(32, 1, 8)
+            RA_ROWS_CASE(64, 1, 8)
+            RA_ROWS_CASE(16, 1, 16)
+            RA_ROWS_CASE(32, 1, 16)
+            RA_ROWS_CASE(64, 1, 16)
+        }
+    }
 #undef RA_ROWS_G
 #undef RA_ROWS_CASE
     return ra::fail(RA_ERR_INTERNAL, "csr_rows: no lane shape");
 }
 
-template <typename P>
+template <typename P, typename Rows>
 ra_status launch_zo(const LaneShape& sh, dim3 grid, hipStream_t st, const int32_t* rowptr,
-                    const int32_t* colind, const float* vals, const P* B, P* C,
+                    const int32_t* colind, const float* vals, const float* B, float* C,
                     const int32_t* chunk_rows, const int32_t* chunk_starts,
-                    const int32_t* chunk_slot, int num_chunks, P* partials,
-                    const int32_t* short_rows, int64_t num_short, int64_t ldp, int np,
-                    bool xcd_slices) {
-    const int remap = tuning().zo_remap, nt = tuning().nt, sole_split = tuning().sole_split;
+                    const int32_t* chunk_slot, int num_chunks, float* partials,
+                    const int32_t* short_rows, int64_t num_short, int N, bool xcd_slices) {
+    const int remap = tuning().zo_remap, nt = tuning().nt && whole_packets(C, N), sole_split = tuning().sole_split;
     int nslices = 0;
     if (xcd_slices && grid.y > 1 && fold_fits(grid)) {  // same 2^32 work-item bound
         nslices = static_cast<int>(grid.y);
@@ -638,23 +753,32 @@ ra_status launch_zo(const LaneShape& sh, dim3 grid, hipStream_t st, const int32_
     }
 #define RA_ZO_CASE(g, v, u)                                                                  \
     if (sh.G == g && sh.V == v && sh.U == u) {                                               \
-        zo_fused_kernel<g, v, u, P><<<grid, kBlock, 0, st>>>(                                \
+        zo_fused_kernel<g, v, u, P, Rows><<<grid, kBlock, 0, st>>>(                          \
             rowptr, colind, vals, B, C, chunk_rows, chunk_starts, chunk_slot, num_chunks,    \
-            partials, short_rows, num_short, ldp, np, remap, nt, sole_split, nslices,        \
+            partials, short_rows, num_short, N, remap, nt, sole_split, nslices,              \
             tuning().lds_stage);                                                             \
         RA_LAUNCH_CHECK("zo_fused_kernel");                                                  \
         return RA_OK;                                                                        \
     }
 #define RA_ZO_G(g, u) RA_ZO_CASE(g, 1, u) RA_ZO_CASE(g, 2, u) RA_ZO_CASE(g, 4, u)
-    RA_ZO_G(4, 4)
-    RA_ZO_G(8, 4)
-    RA_ZO_G(8, 8)
-    RA_ZO_G(16, 4)
-    RA_ZO_G(16, 8)
-    RA_ZO_G(32, 4)
-    RA_ZO_G(32, 8)
-    RA_ZO_G(64, 4)
-    RA_ZO_G(64, 8)
+    RA_ZO_CASE(4, 1, 4)
+    if constexpr (PacketElems<P>::value == 4) {
+        RA_ZO_CASE(4, 2, 4)
+        RA_ZO_CASE(4, 4, 4)
+        RA_ZO_G(8, 4)
+        RA_ZO_G(16, 4)
+        RA_ZO_G(32, 4)
+        RA_ZO_G(64, 4)
+        if constexpr (std::is_same_v<Rows, BufferRows>) {
+            RA_ZO_CASE(8, 1, 8)
+            RA_ZO_CASE(16, 1, 8)
+            RA_ZO_CASE(32, 1, 8)
+            RA_ZO_CASE(64, 1, 8)
+            RA_ZO_CASE(16, 1, 16)
+            RA_ZO_CASE(32, 1, 16)
+            RA_ZO_CASE(64, 1, 16)
+        }
+    }
 #undef RA_ZO_G
 #undef RA_ZO_CASE
     return ra::fail(RA_ERR_INTERNAL, "zo: no lane shape");
@@ -684,8 +808,8 @@ ra_status csr_direct_launch(const int32_t* d_rowptr, const int32_t* d_colind, co
                             bool resume, hipStream_t st) {
     RA_TRY(check_spmm_args(d_rowptr, d_colind, d_vals, d_B, d_C, M, K, N, nnz));
     if (M == 0 || N == 0) return RA_OK;
-    const bool vec = (N % 4 == 0) && ra::aligned16(d_B) && ra::aligned16(d_C);
-    const int np = vec ? N / 4 : N;
+    const bool vec = N >= 4;
+    const int np = vec ? (N + 3) / 4 : N;
     // Wide rows of a small matrix: 128-column slices dealt to the XCDs, as
     // ZERO_OVERHEAD_CSR does, so that fewer than 2^16 waves (about 64 per CU)
     // become 2-4x as many, each with a shorter chain of dependent gathers.
@@ -697,17 +821,15 @@ ra_status csr_direct_launch(const int32_t* d_rowptr, const int32_t* d_colind, co
         const int64_t waves = (static_cast<int64_t>(M) + kWave / whole.G - 1) / (kWave / whole.G);
         cslice = (vec && N >= 256 && waves < (int64_t{1} << 16)) ? 128 : 0;
     }
-    const LaneShape sh = pick_shape(np, vec ? 4 : 1, cslice);
+    LaneShape sh = pick_shape(np, vec ? 4 : 1, cslice);
     const bool deal = cslice > 0 || tuning().xslice;
     const int rows_per_block = kWavesPerBlock * (kWave / sh.G);
     dim3 grid((M + rows_per_block - 1) / rows_per_block, (np + sh.G * sh.V - 1) / (sh.G * sh.V));
-    if (vec)
-        return launch_csr_rows<float4>(sh, grid, st, d_rowptr, d_colind, d_vals,
-                                       reinterpret_cast<const float4*>(d_B),
-                                       reinterpret_cast<float4*>(d_C), nullptr, M, np, np, resume ? 1 : 0,
-                                       deal);
-    return launch_csr_rows<float>(sh, grid, st, d_rowptr, d_colind, d_vals, d_B, d_C,
-                                  nullptr, M, np, np, resume ? 1 : 0, deal);
+    const bool buf = buffer_rows_fit(K, N);
+    if (buf && vec) sh.U = gathers_in_flight(sh, (int64_t)grid.x * grid.y * kWavesPerBlock);
+    auto launch = vec ? (buf ? launch_csr_rows<pk4, BufferRows> : launch_csr_rows<pk4, PointerRows>)
+                      : (buf ? launch_csr_rows<float, BufferRows> : launch_csr_rows<float, PointerRows>);
+    return launch(sh, grid, st, d_rowptr, d_colind, d_vals, d_B, d_C, M, N, resume ? 1 : 0, deal);
 }
 
 }  // namespace ra
@@ -722,12 +844,12 @@ static ra_status zo_run(ra_zo_plan* plan, const int32_t* d_rowptr, const int32_t
     const int32_t M = plan->info.M;
     RA_TRY(check_spmm_args(d_rowptr, d_colind, d_vals, d_B, d_C, M, plan->info.K, N, 0));
     if (M == 0 || N == 0) return RA_OK;
-    const bool vec = (N % 4 == 0) && ra::aligned16(d_B) && ra::aligned16(d_C);
-    const int np = vec ? N / 4 : N;
+    const bool vec = N >= 4;
+    const int np = vec ? (N + 3) / 4 : N;
     // Wide rows are cut into 128-column slices dealt to the XCDs (each XCD's
     // L2 then holds half or less of every gathered B row).
     const int zslice = tuning().zo_slice >= 0 ? tuning().zo_slice : (vec && N >= 256 ? 128 : 0);
-    const LaneShape sh = pick_shape(np, vec ? 4 : 1, zslice);
+    LaneShape sh = pick_shape(np, vec ? 4 : 1, zslice);
     if (plan->info.num_split_chunks > 0 && !partials) {
         RA_TRY(plan->partials.ensure((size_t)plan->info.num_split_chunks * N * sizeof(float)));
         partials = plan->partials.get<float>();
@@ -737,34 +859,19 @@ static ra_status zo_run(ra_zo_plan* plan, const int32_t* d_rowptr, const int32_t
     const int tiles = (np + sh.G * sh.V - 1) / (sh.G * sh.V);
     if (waves > 0 && stage != 2) {
         dim3 grid((waves + kWavesPerBlock - 1) / kWavesPerBlock, tiles);
-        ra_status s;
-        if (vec)
-            s = launch_zo<float4>(sh, grid, st, d_rowptr, d_colind, d_vals,
-                                  reinterpret_cast<const float4*>(d_B), reinterpret_cast<float4*>(d_C),
-                                  plan->chunk_rows, plan->chunk_starts,
-                                  plan->chunk_slot, plan->info.num_chunks,
-                                  reinterpret_cast<float4*>(partials), plan->short_rows,
-                                  plan->num_short_total, np, np, zslice > 0);
-        else
-            s = launch_zo<float>(sh, grid, st, d_rowptr, d_colind, d_vals, d_B, d_C,
-                                 plan->chunk_rows, plan->chunk_starts,
-                                 plan->chunk_slot, plan->info.num_chunks,
-                                 partials, plan->short_rows,
-                                 plan->num_short_total, np, np, zslice > 0);
-        RA_TRY(s);
+        const bool buf = buffer_rows_fit(plan->info.K, N);
+        if (buf && vec) sh.U = gathers_in_flight(sh, waves * tiles);
+        auto launch = vec ? (buf ? launch_zo<pk4, BufferRows> : launch_zo<pk4, PointerRows>)
+                          : (buf ? launch_zo<float, BufferRows> : launch_zo<float, PointerRows>);
+        RA_TRY(launch(sh, grid, st, d_rowptr, d_colind, d_vals, d_B, d_C, plan->chunk_rows, plan->chunk_starts,
+                      plan->chunk_slot, plan->info.num_chunks, partials, plan->short_rows, plan->num_short_total,
+                      N, zslice > 0));
     }
     if (plan->info.num_split_rows > 0 && stage != 1) {
         const int64_t threads = (int64_t)plan->info.num_split_rows * np;
         const unsigned grid = static_cast<unsigned>((threads + kBlock - 1) / kBlock);
-        if (vec)
-            zo_merge_kernel<float4><<<grid, kBlock, 0, st>>>(
-                plan->split_rows, plan->split_off,
-                reinterpret_cast<float4*>(partials), reinterpret_cast<float4*>(d_C), np, np,
-                plan->info.num_split_rows);
-        else
-            zo_merge_kernel<float><<<grid, kBlock, 0, st>>>(
-                plan->split_rows, plan->split_off,
-                partials, d_C, np, np, plan->info.num_split_rows);
+        (vec ? zo_merge_kernel<pk4> : zo_merge_kernel<float>)<<<grid, kBlock, 0, st>>>(
+            plan->split_rows, plan->split_off, partials, d_C, N, np, plan->info.num_split_rows);
         RA_LAUNCH_CHECK("zo_merge_kernel");
     }
     return RA_OK;
