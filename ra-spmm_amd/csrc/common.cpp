@@ -1,6 +1,9 @@
-// common.cpp — error state, names and the host parallel_for of the C ABI.
+// common.cpp — error state, names, the host parallel_for and the device memory
+// pool of the C ABI.
 #include <algorithm>
 #include <atomic>
+#include <map>
+#include <mutex>
 #include <thread>
 
 #include "ra_internal.hpp"
@@ -41,9 +44,138 @@ void parallel_for(int64_t n, int64_t grain, const std::function<void(int64_t, in
     for (auto& t : pool) t.join();
 }
 
+// ------------------------------------------------------- device memory pool
+namespace {
+
+struct PoolBlock {
+    void* ptr;
+    uint64_t age;
+};
+
+struct DevicePool {
+    std::multimap<size_t, PoolBlock> free_blocks;  // by capacity
+    size_t held = 0;
+};
+
+struct Pool {
+    std::mutex mutex;
+    std::map<int, DevicePool> devices;
+    uint64_t clock = 0;
+};
+
+// Never destroyed: plans may outlive static destructors, and the runtime frees
+// the memory at exit.
+Pool& pool() {
+    static Pool* p = new Pool();
+    return *p;
+}
+
+// Eight classes per power of two: at most 1/8 is wasted, and plans of graphs of
+// about the same size use each other's blocks.
+size_t size_class(size_t bytes) {
+    size_t power = 4096;
+    while (power * 2 <= bytes) power *= 2;
+    const size_t step = power / 8;
+    return (bytes + step - 1) / step * step;
+}
+
+// Current device switched for one scope.
+class OnDevice {
+public:
+    explicit OnDevice(int device) {
+        (void)hipGetDevice(&old_);
+        if (old_ != device) (void)hipSetDevice(device);
+        switched_ = old_ != device;
+    }
+    ~OnDevice() {
+        if (switched_) (void)hipSetDevice(old_);
+    }
+
+private:
+    int old_ = 0;
+    bool switched_ = false;
+};
+
+// Free the blocks of `d` from the oldest on until at most `keep` bytes are held.
+void trim_locked(int device, DevicePool& d, size_t keep) {
+    if (d.held <= keep) return;
+    const OnDevice on(device);
+    while (d.held > keep && !d.free_blocks.empty()) {
+        auto oldest = d.free_blocks.begin();
+        for (auto it = d.free_blocks.begin(); it != d.free_blocks.end(); ++it)
+            if (it->second.age < oldest->second.age) oldest = it;
+        (void)hipFree(oldest->second.ptr);
+        d.held -= oldest->first;
+        d.free_blocks.erase(oldest);
+    }
+}
+
+}  // namespace
+
+ra_status pool_allocate(void** ptr, size_t bytes, size_t* capacity, int* device) {
+    *ptr = nullptr;
+    RA_HIP_TRY(hipGetDevice(device));
+    const size_t want = size_class(bytes);
+    Pool& p = pool();
+    {
+        std::lock_guard<std::mutex> lock(p.mutex);
+        DevicePool& d = p.devices[*device];
+        const auto it = d.free_blocks.lower_bound(want);
+        if (it != d.free_blocks.end() && it->first <= want + want / 4) {
+            *ptr = it->second.ptr;
+            *capacity = it->first;
+            d.held -= it->first;
+            d.free_blocks.erase(it);
+            return RA_OK;
+        }
+    }
+    hipError_t e = hipMalloc(ptr, want);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        {
+            std::lock_guard<std::mutex> lock(p.mutex);
+            trim_locked(*device, p.devices[*device], 0);
+        }
+        e = hipMalloc(ptr, want);
+    }
+    if (e != hipSuccess) {
+        *ptr = nullptr;
+        return hip_fail(e, "hipMalloc");
+    }
+    *capacity = want;
+    return RA_OK;
+}
+
+void pool_release(void* ptr, size_t capacity, int device, bool idle) {
+    {
+        // What cannot be waited for (a stream of this thread is being captured)
+        // is not reused.
+        const OnDevice on(device);
+        if (capacity > kPoolBytes || (!idle && hipDeviceSynchronize() != hipSuccess)) {
+            (void)hipGetLastError();
+            (void)hipFree(ptr);
+            return;
+        }
+    }
+    Pool& p = pool();
+    std::lock_guard<std::mutex> lock(p.mutex);
+    DevicePool& d = p.devices[device];
+    d.free_blocks.emplace(capacity, PoolBlock{ptr, ++p.clock});
+    d.held += capacity;
+    trim_locked(device, d, kPoolBytes);
+}
+
+void pool_trim() {
+    Pool& p = pool();
+    std::lock_guard<std::mutex> lock(p.mutex);
+    for (auto& d : p.devices) trim_locked(d.first, d.second, 0);
+}
+
 }  // namespace ra
 
 extern "C" {
+
+void ra_release_memory(void) { ra::pool_trim(); }
 
 int ra_abi_version(void) { return RA_SPMM_ABI_VERSION; }
 

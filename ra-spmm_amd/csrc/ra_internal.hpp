@@ -49,14 +49,30 @@ inline ra_status hip_fail(hipError_t e, const char* what) {
         if (_e != hipSuccess) return ::ra::hip_fail(_e, what);       \
     } while (0)
 
-// Owning device allocation (hipMalloc / hipFree).
+// Device memory kept between plans (common.cpp): a block given back stays
+// allocated, up to kPoolBytes per device, and serves a later request of its
+// size class.  hipMalloc and hipFree of a tile plan and its build scratch (1.4
+// GB for 512,000 rows and 1.6e7 nonzeros) cost a one-off call 10 to 40 ms
+// against 3 ms of kernels; from the pool they cost nothing.
+//
+// Streams and threads: a block enters the pool only once nothing on the device
+// can still be using it, as hipFree would wait for (`idle` says that the caller
+// has waited already), so the next owner may use it on any stream.  The lists
+// are locked.  Memory goes back to the driver when the pool is full (oldest
+// block first), when an allocation fails, and on pool_trim().
+constexpr size_t kPoolBytes = size_t(4) << 30;
+ra_status pool_allocate(void** ptr, size_t bytes, size_t* capacity, int* device);
+void pool_release(void* ptr, size_t capacity, int device, bool idle);
+void pool_trim();
+
+// Owning device allocation, from the pool.
 class DeviceBuffer {
 public:
     DeviceBuffer() = default;
     ~DeviceBuffer() { reset(); }
     DeviceBuffer(const DeviceBuffer&) = delete;
     DeviceBuffer& operator=(const DeviceBuffer&) = delete;
-    DeviceBuffer(DeviceBuffer&& o) noexcept : ptr_(o.ptr_), bytes_(o.bytes_) {
+    DeviceBuffer(DeviceBuffer&& o) noexcept : ptr_(o.ptr_), bytes_(o.bytes_), device_(o.device_) {
         o.ptr_ = nullptr;
         o.bytes_ = 0;
     }
@@ -65,6 +81,7 @@ public:
             reset();
             std::swap(ptr_, o.ptr_);
             std::swap(bytes_, o.bytes_);
+            std::swap(device_, o.device_);
         }
         return *this;
     }
@@ -80,13 +97,7 @@ public:
                 return fail(RA_ERR_OUT_OF_MEMORY, "hipMalloc: " + std::to_string(bytes) +
                                                       " bytes exceed RA_MAX_ALLOC_BYTES");
         }
-        hipError_t e = hipMalloc(&ptr_, bytes);
-        if (e != hipSuccess) {
-            ptr_ = nullptr;
-            return hip_fail(e, "hipMalloc");
-        }
-        bytes_ = bytes;
-        return RA_OK;
+        return pool_allocate(&ptr_, bytes, &bytes_, &device_);
     }
     // Grow-only reuse (plan scratch).
     ra_status ensure(size_t bytes) {
@@ -102,18 +113,22 @@ public:
         }
         return RA_OK;
     }
-    void reset() {
-        if (ptr_) (void)hipFree(ptr_);
-        ptr_ = nullptr;
-        bytes_ = 0;
-    }
+    void reset() { release(false); }
+    // As reset(), where the caller has waited for everything that used it.
+    void reset_idle() { release(true); }
     template <typename T = void>
     T* get() const { return static_cast<T*>(ptr_); }
     size_t bytes() const { return bytes_; }
 
 private:
+    void release(bool idle) {
+        if (ptr_) pool_release(ptr_, bytes_, device_, idle);
+        ptr_ = nullptr;
+        bytes_ = 0;
+    }
     void* ptr_ = nullptr;
     size_t bytes_ = 0;
+    int device_ = 0;
 };
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

@@ -635,6 +635,8 @@ ra_status gpu_build(ra_tile_plan* p, int32_t kind, const int32_t* rowptr, const 
         RA_TRY(read_back(&p->part_splits[q], split_idx + (int64_t)q * W, 1, st));
     }
 
+    s.buf.reset_idle();  // the last read-back waited for the stream, which alone used it
+
     ra_tile_info& I = p->info;
     I.active = 1;
     I.col_parts = P;

@@ -809,4 +809,6 @@ PYBIND11_MODULE(_C, m) {
           "Diagnostic structural features of a CSR matrix (host computation)", pybind11::arg("rowptr"),
           pybind11::arg("colind"), pybind11::arg("M"), pybind11::arg("K"), pybind11::arg("N"));
     m.def("abi_version", &ra_abi_version);
+    m.def("release_memory", &ra_release_memory,
+          "Give the device memory kept from destroyed plans back to the driver");
 }

@@ -25,8 +25,7 @@ constexpr uint32_t kSoleFlag = 0x80000000u;
 struct ra_zo_plan {
     ra_zo_info info{};
     int device = 0;
-    // The six lists live in one allocation (one hipMalloc per build, one
-    // hipFree per plan): short_rows | chunk_rows | chunk_starts | chunk_slot |
+    // The six lists live in one allocation: short_rows | chunk_rows | chunk_starts | chunk_slot |
     // split_rows | split_off, each 256-byte aligned.
     ra::DeviceBuffer lists;
     int32_t *short_rows = nullptr, *chunk_rows = nullptr, *chunk_starts = nullptr, *chunk_slot = nullptr,

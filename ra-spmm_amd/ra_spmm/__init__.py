@@ -20,7 +20,7 @@ except ImportError as exc:  # pragma: no cover - exercised only on broken instal
 from ._C import (  # noqa: F401
     CuSparsePlan, RACommunityTCPlan, analyze_matrix, RASegmentHybridPlan, RATcDirectPlan, RATilePlan,
     RAZeroOverheadPlan, compute_features, export_tile_plan, export_zero_overhead_plan, make_community_tc_plan, make_cusparse_plan,
-    make_router_plan, make_segment_hybrid_plan, make_tc_direct_plan, make_zero_overhead_plan,
+    make_router_plan, make_segment_hybrid_plan, make_tc_direct_plan, make_zero_overhead_plan, release_memory,
     route_features, run_community_tc_plan, run_community_tc_plan_tf32, run_cusparse_plan,
     run_segment_hybrid_plan, run_segment_hybrid_plan_tf32, run_tc_direct_plan,
     run_tc_direct_plan_tf32, run_tile_plan_route, run_zero_overhead_plan, spmm_csr_baseline,

@@ -19,7 +19,7 @@ TABLE_REFERENCE, TABLE_MI355X = 0, 1
 
 # Every function include/ra_spmm.h declares (checked by tests/test_capi_symbols.py).
 EXPORTED = [
-    "ra_abi_version", "ra_status_string", "ra_last_error", "ra_path_name", "ra_reject_name",
+    "ra_abi_version", "ra_release_memory", "ra_status_string", "ra_last_error", "ra_path_name", "ra_reject_name",
     "ra_features_host", "ra_features_device", "ra_features_from_moments", "ra_route_dispatch",
     "ra_analyze_matrix",
     "ra_spmm_csr_direct", "ra_spmm_csr_baseline", "ra_spmm_csr_baseline_f16", "ra_zo_bins_host", "ra_zo_plan_create",
@@ -125,6 +125,7 @@ def load():
     I32, I64 = ctypes.c_int32, ctypes.c_int64
     sig = {
         "ra_abi_version": (ctypes.c_int, []),
+        "ra_release_memory": (None, []),
         "ra_status_string": (ctypes.c_char_p, [ctypes.c_int]),
         "ra_last_error": (ctypes.c_char_p, []),
         "ra_path_name": (ctypes.c_char_p, [I32]),

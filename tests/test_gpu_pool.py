@@ -1,0 +1,71 @@
+"""Device memory kept between plans: reused, bounded, given back, and never
+handed on while a stream may still be using it."""
+import threading
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+import ra_spmm  # noqa: E402
+from ra_spmm import synthetic as S  # noqa: E402
+
+
+def _free():
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    return torch.cuda.mem_get_info()[0] + torch.cuda.memory_reserved()
+
+
+def test_reuse_and_release():
+    g = S.sbm(256, 100, 24.0, 0.9, seed=2)
+    rp, ci, vl = g.torch("cuda")
+    B = torch.randn(g.K, 64, device="cuda")
+
+    def once():
+        plan = ra_spmm.make_tc_direct_plan(rp, ci, vl, g.M, g.K, 64)
+        return ra_spmm.run_tc_direct_plan(plan, B)
+
+    ref = once()
+    _free()
+    assert torch.equal(once(), ref)  # the one-time allocations of the runtime are done after this
+    kept = _free()
+    for _ in range(4):
+        assert torch.equal(once(), ref)
+    assert abs(_free() - kept) < (2 << 20)
+    ra_spmm.release_memory()
+    assert _free() - kept > (1 << 20)  # the blocks of the dead plans went back
+    assert torch.equal(once(), ref)
+
+
+def test_plans_of_other_streams_and_threads():
+    """A plan dropped right after its run was queued on a side stream: the next plans, on other streams and threads,
+    must not get its memory before the run is done."""
+    graphs = [S.random_csr(4000, 4000, 20.0 + i, seed=i, skew=1.2) for i in range(3)]
+    inputs = []
+    for i, g in enumerate(graphs):
+        rp, ci, vl = g.torch("cuda")
+        B = torch.randn(g.K, 96, device="cuda", generator=torch.Generator("cuda").manual_seed(i))
+        plan = ra_spmm.make_segment_hybrid_plan(rp, ci, vl, g.M, g.K, 96)
+        inputs.append((g, rp, ci, vl, B, ra_spmm.run_segment_hybrid_plan(plan, ci, vl, B)))
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(i):
+        g, rp, ci, vl, B, ref = inputs[i]
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                plan = ra_spmm.make_segment_hybrid_plan(rp, ci, vl, g.M, g.K, 96)
+                out = ra_spmm.run_segment_hybrid_plan(plan, ci, vl, B)
+                del plan
+                stream.synchronize()
+                if not torch.equal(out, ref):
+                    wrong.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not wrong
