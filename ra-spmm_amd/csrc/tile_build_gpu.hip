@@ -295,6 +295,25 @@ __global__ void fill_segments(const int32_t* __restrict__ block_offsets, const i
     }
 }
 
+// Launch order of the items: within every partition the long ones first.
+// rank = exclusive scan of the long flags over all items.
+__global__ void flag_long(const int32_t* __restrict__ bbegin, const int32_t* __restrict__ bend, int64_t n, int limit,
+                          int32_t* __restrict__ flag) {
+    RA_GRID_STRIDE(i, n + 1) flag[i] = i < n && bend[i] - bbegin[i] > limit ? 1 : 0;
+}
+
+__global__ void order_items(const int32_t* __restrict__ flag, const int32_t* __restrict__ rank,
+                            const int32_t* __restrict__ seg_start, int64_t W, int P, int64_t n,
+                            int32_t* __restrict__ order) {
+    RA_GRID_STRIDE(i, n) {
+        int q = 0;
+        while (q + 1 < P && seg_start[(q + 1) * W] <= i) ++q;
+        const int32_t base = seg_start[q * W], end = seg_start[(q + 1) * W];
+        const int32_t before = rank[i] - rank[base], longs = rank[end] - rank[base];
+        order[base + (flag[i] ? before : longs + static_cast<int32_t>(i - base) - before)] = static_cast<int32_t>(i);
+    }
+}
+
 struct Scratch {
     ra::DeviceBuffer buf;
     template <typename T>
@@ -630,9 +649,37 @@ ra_status gpu_build(ra_tile_plan* p, int32_t kind, const int32_t* rowptr, const 
     // partition-major, so each partition's items are one contiguous run).
     p->part_items.assign(P + 1, 0);
     p->part_splits.assign(P + 1, 0);
-    for (int q = 1; q <= P; ++q) {
+    for (int q = 1; q < P; ++q) {
         RA_TRY(read_back(&p->part_items[q], seg_start + (int64_t)q * W, 1, st));
         RA_TRY(read_back(&p->part_splits[q], split_idx + (int64_t)q * W, 1, st));
+    }
+    p->part_items[P] = static_cast<int32_t>(nseg);
+    p->part_splits[P] = static_cast<int32_t>(nsplit);
+
+    // Launch order, where some item is long (128 blocks of 8 vectors).
+    p->part_long.assign(P, 0);
+    const int long_blocks = ra::kTileLongBlocks * ra::kTileVec / L.vb;
+    p->has_long = reds[0] > long_blocks;
+    if (p->has_long) {
+        size_t scan6 = 0;
+        RA_HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, scan6, inull, inull, static_cast<int>(nseg + 1), st));
+        ra::DeviceBuffer ranks, scan_tmp;
+        RA_TRY(ranks.allocate(2 * (nseg + 1) * sizeof(int32_t)));
+        RA_TRY(scan_tmp.allocate(scan6));
+        RA_TRY(p->item_order.allocate(nseg * sizeof(int32_t)));
+        int32_t *flag = ranks.get<int32_t>(), *rank = flag + nseg + 1;
+        flag_long<<<grid_for(nseg + 1), kThreads, 0, st>>>(p->seg_bbegin.get<int32_t>(), p->seg_bend.get<int32_t>(),
+                                                           nseg, long_blocks, flag);
+        RA_HIP_TRY(hipcub::DeviceScan::ExclusiveSum(scan_tmp.get(), scan6, flag, rank, static_cast<int>(nseg + 1), st));
+        order_items<<<grid_for(nseg), kThreads, 0, st>>>(flag, rank, seg_start, W, P, nseg,
+                                                         p->item_order.get<int32_t>());
+        RA_LAUNCH_CHECK("order_items");
+        std::vector<int32_t> at(P + 1);
+        for (int q = 0; q <= P; ++q) RA_TRY(read_back(&at[q], rank + p->part_items[q], 1, st));
+        for (int q = 0; q < P; ++q) p->part_long[q] = at[q + 1] - at[q];
+        RA_HIP_TRY(hipStreamSynchronize(st));
+        ranks.reset_idle();
+        scan_tmp.reset_idle();
     }
 
     s.buf.reset_idle();  // the last read-back waited for the stream, which alone used it

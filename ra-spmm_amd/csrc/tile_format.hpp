@@ -44,6 +44,9 @@ constexpr int kTileSegBlocks = 64;    // SEGMENT_HYBRID: max blocks per segment
 // thousands of blocks while the rest of the GPU idles.
 constexpr int kTileDirectSplitBlocks = 512;
 constexpr uint32_t kTileSoleFlag = 0x80000000u;
+// Items (segments) of more blocks than this are run first, each by a whole
+// workgroup.
+constexpr int kTileLongBlocks = 128;
 
 uint16_t f32_to_f16_rne(float f);
 // Power-of-two scale 2^s for fp16 storage: maps max|v| near 2^14 so small
@@ -68,6 +71,11 @@ struct ra_tile_plan {
     // partition q are [part_items[q], part_items[q+1]) and
     // [part_splits[q], part_splits[q+1]); cells are q * num_windows + window.
     std::vector<int32_t> part_items{0, 0}, part_splits{0, 0};
+    // Items of every partition in launch order: the part_long[q] long ones
+    // first, otherwise ascending.  Used where has_long.
+    ra::DeviceBuffer item_order;
+    std::vector<int32_t> part_long{0};
+    bool has_long = false;
     ra::DeviceBuffer bconv;    // B converted to fp16/bf16 (grown per K*ldb)
     ra::DeviceBuffer scratch;  // partial slots of split windows
     // FP32 route: the stored values as a CSR sorted by (row, column), derived

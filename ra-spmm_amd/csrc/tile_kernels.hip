@@ -4,7 +4,8 @@
 // (SEGMENT_HYBRID): 8 output rows and a run of blocks [b0, b1).
 //
 // FP16/BF16 route (tile_mfma_kernel): one wavefront per (item, 16*CPL-column
-// slice), v_mfma_f32_16x16x32_{f16,bf16}.  A step consumes 4 blocks (32
+// slice), or a workgroup where the item is long or the launch small
+// (shared_items), v_mfma_f32_16x16x32_{f16,bf16}.  A step consumes 4 blocks (32
 // vectors = the MFMA K).  Lane (j = lane & 15, q = lane >> 4):
 //   - gathers B rows atox[(b+q)*8 + v], v < 8, CPL contiguous elements each at
 //     columns col0 + j*CPL (one 16-byte load per vector for CPL = 8), then
@@ -66,14 +67,94 @@ __device__ __forceinline__ f32x4 mfma32(u16x8 a, u16x8 b, f32x4 c) {
                                                       __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
+// Where the gathered rows of the 16-bit B are.  A column index becomes a key
+// before the lanes hand it to each other; -1 (padding of a window's last block)
+// gathers zeros.
+//
+// HalfBuffer: key = byte offset of the row, gathered through a buffer
+// descriptor of K rows: the offset of row -1 lies past its end, where the
+// bounds check returns 0.  A step's eight gathers then leave back to back; with
+// a branch around each the compiler waits for earlier loads in between: 512,000
+// community rows at N = 512 1,215 -> 1,157 us, 64,000 at N = 128 48.3 -> 43.4,
+// 150,000 social rows of 200 at N = 128 769 -> 690, 50,000 of 80 109 -> 91.
+// HalfPointer: 64-bit addresses, for a B of 4 GiB and more.
+template <int CPL>
+struct HalfBuffer {
+    typedef typename HalfRun<CPL>::T Run;
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t row_bytes, col_bytes;
+    __device__ __forceinline__ HalfBuffer(const uint16_t* Bh, int K, int ldb, int col)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(Bh), 0,
+                                                 static_cast<int>(static_cast<uint32_t>(K) * (ldb * 2u)), 0x00027000)),
+          row_bytes(ldb * 2u), col_bytes(col * 2u) {}
+    __device__ __forceinline__ int key(int col) const { return static_cast<int>(static_cast<uint32_t>(col) * row_bytes); }
+    __device__ __forceinline__ Run load(int key) const {
+        const uint32_t off = static_cast<uint32_t>(key) + col_bytes;
+        if constexpr (CPL == 8)
+            return __builtin_bit_cast(Run, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
+        else if constexpr (CPL == 4)
+            return __builtin_bit_cast(Run, __builtin_amdgcn_raw_buffer_load_b64(rsrc, off, 0, 0));
+        else if constexpr (CPL == 2)
+            return __builtin_bit_cast(Run, __builtin_amdgcn_raw_buffer_load_b32(rsrc, off, 0, 0));
+        else
+            return __builtin_amdgcn_raw_buffer_load_b16(rsrc, off, 0, 0);
+    }
+};
+
+template <int CPL>
+struct HalfPointer {
+    typedef typename HalfRun<CPL>::T Run;
+    const uint16_t* base;
+    int64_t ldb;
+    __device__ __forceinline__ HalfPointer(const uint16_t* Bh, int, int ld, int col) : base(Bh + col), ldb(ld) {}
+    __device__ __forceinline__ int key(int col) const { return col; }
+    __device__ __forceinline__ Run load(int key) const {
+        return key >= 0 ? *reinterpret_cast<const Run*>(base + key * ldb) : Run{};
+    }
+};
+
+// Index chunk of a lane: four consecutive column indices, -1 past the item.
+// They become keys when their steps begin, not when they are loaded (a chunk
+// ahead): the loop does not wait for the load.
+__device__ __forceinline__ int4 load_chunk4(const int32_t* __restrict__ atox, int64_t at, bool inside) {
+    int4 v = make_int4(-1, -1, -1, -1);
+    if (inside) v = *reinterpret_cast<const int4*>(atox + at);
+    return v;
+}
+template <typename BRows>
+__device__ __forceinline__ int4 chunk_keys(const BRows& rows, const int4& v) {
+    return make_int4(rows.key(v.x), rows.key(v.y), rows.key(v.z), rows.key(v.w));
+}
+
+// The eight keys held by lanes l0 and l0 + 1.
+__device__ __forceinline__ void share_keys(const int4& chunk, int l0, int (&keys)[8]) {
+    keys[0] = __shfl(chunk.x, l0, kWave);
+    keys[1] = __shfl(chunk.y, l0, kWave);
+    keys[2] = __shfl(chunk.z, l0, kWave);
+    keys[3] = __shfl(chunk.w, l0, kWave);
+    keys[4] = __shfl(chunk.x, l0 + 1, kWave);
+    keys[5] = __shfl(chunk.y, l0 + 1, kWave);
+    keys[6] = __shfl(chunk.z, l0 + 1, kWave);
+    keys[7] = __shfl(chunk.w, l0 + 1, kWave);
+}
+
+// The lane's eight gathers of a step.
+template <typename BRows, typename Run>
+__device__ __forceinline__ void gather8(const BRows& rows, const int (&keys)[8], Run (&raw)[8]) {
+#pragma unroll
+    for (int v = 0; v < 8; ++v) raw[v] = rows.load(keys[v]);
+}
+
 struct Items {
     const int32_t* block_offsets;
     const int32_t* seg_window;
     const int32_t* seg_bbegin;
     const int32_t* seg_bend;
     const int32_t* seg_slot;
-    const int32_t* win_rows;       // COMMUNITY_TC
+    const int32_t* win_rows;       // COMMUNITY_TC's row order, NULL for rows in order
+    const int32_t* order;          // items of this launch, the long ones first (NULL: in order)
     int item_base;                 // first segment of this launch
+    int num_long;                  // items that a whole workgroup shares
     int cell_base;                 // partition * windows (column partitions)
     int accumulate;                // add into C (partitions after the first)
 };
@@ -93,6 +174,7 @@ __device__ __forceinline__ void put4(float* dst, V4 v, bool add) {
 __device__ __forceinline__ void item_range(const Items& it, int i, int& w, int& b0, int& b1,
                                            int& slot) {
     i += it.item_base;
+    if (it.order) i = it.order[i];
     w = static_cast<int>(static_cast<uint32_t>(it.seg_window[i]) & 0x7FFFFFFFu) - it.cell_base;
     b0 = it.seg_bbegin[i];
     b1 = it.seg_bend[i];
@@ -100,68 +182,129 @@ __device__ __forceinline__ void item_range(const Items& it, int i, int& w, int& 
 }
 
 // Destination of window slot m (0..H-1): a C row, or a partial-slot row.
-template <int KIND, int H = ra::kTileWindow>
+template <int H = ra::kTileWindow>
 __device__ __forceinline__ float* item_row(const Items& it, float* C, float* scratch, int w,
                                            int slot, int m, int M, int N) {
     if (slot >= 0) return scratch + ((int64_t)slot * H + m) * N;
-    int row;
-    if constexpr (KIND == RA_TILE_COMMUNITY_TC) row = it.win_rows[(int64_t)w * H + m];
-    else row = w * H + m;
+    const int row = it.win_rows ? it.win_rows[(int64_t)w * H + m] : w * H + m;
     if (row < 0 || row >= M) return nullptr;
     return C + (int64_t)row * N;
 }
 
-// 1-D grid: block -> (group of 4 items, column slice), slice fastest, so all
-// slices of a window run back to back and share its atox/vals in L2.  With
-// remap on, each XCD (workgroups are dealt round-robin over 8) takes one
-// contiguous range of windows, keeping neighbouring windows in one L2.
-// order bit 0: XCD remap; bit 1: slice slowest (all windows of slice 0, then
+// What a wave runs: blocks [b0, b1) of one item, in one column slice.
+struct WaveWork {
+    int slice, w, b0, b1, slot;
+    bool shared;  // a quarter of the item; the workgroup's waves sum up
+};
+
+// 1-D grid of workgroups: num_long * nslices that share one item each, then
+// groups of 4 items, one a wave.  The slice runs fastest, so all slices of a
+// window run back to back and share its atox/vals in L2.
+// order bit 0: each XCD (workgroups are dealt round-robin over 8) takes one
+// contiguous range of the groups of 4, keeping neighbouring windows in one L2;
+// shared items stay dealt.  Bit 1: slice slowest (all windows of slice 0, then
 // slice 1, ...), which shrinks the gathered working set to one slice of each
 // B row when B is far larger than the L2.
-__device__ __forceinline__ void tile_block_coords(int nslices, int order, int64_t& item_blk,
-                                                  int& slice) {
-    int64_t bid = blockIdx.x;
-    if (order & 1) {
-        const int64_t nb = gridDim.x, q = nb / 8, r = nb % 8, x = bid % 8, k = bid / 8;
-        bid = x < r ? x * (q + 1) + k : r * (q + 1) + (x - r) * q + k;
-    }
-    if (order & 2) {
-        const int64_t per_slice = gridDim.x / nslices;
-        slice = static_cast<int>(bid / per_slice);
-        item_blk = bid - (int64_t)slice * per_slice;
+// A shared item is cut into quarters of whole steps of `step` blocks.  False:
+// nothing to do (for the whole workgroup, where it is shared).
+__device__ __forceinline__ bool wave_work(const Items& it, int num_items, int nslices, int order, int step,
+                                          WaveWork& k) {
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const uint32_t ns = static_cast<uint32_t>(nslices), head = it.num_long * ns;
+    uint32_t bid = blockIdx.x;
+    k.shared = bid < head;
+    int item;
+    if (k.shared) {
+        item = static_cast<int>(bid / ns);
+        k.slice = static_cast<int>(bid - item * ns);
     } else {
-        item_blk = bid / nslices;
-        slice = static_cast<int>(bid - item_blk * nslices);
+        bid -= head;
+        const uint32_t nb = gridDim.x - head;
+        if (order & 1) {
+            const uint32_t q = nb / 8, r = nb % 8, x = bid % 8, i = bid / 8;
+            bid = x < r ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
+        }
+        const uint32_t n = (order & 2) ? nb / ns : ns;
+        const uint32_t hi = bid / n, lo = bid - hi * n;
+        k.slice = static_cast<int>((order & 2) ? hi : lo);
+        item = it.num_long + static_cast<int>((order & 2) ? lo : hi) * kWavesPerBlock + wave;
+    }
+    if (item >= num_items) return false;
+    item_range(it, item, k.w, k.b0, k.b1, k.slot);
+    if (k.shared) {
+        const int steps = (k.b1 - k.b0 + step - 1) / step;
+        const int per = (steps + kWavesPerBlock - 1) / kWavesPerBlock * step;
+        k.b0 += wave * per;
+        k.b1 = min(k.b0 + per, k.b1);
+    }
+    return true;
+}
+
+// Write one window row's CPL columns from col on (16-byte streaming stores where
+// the rows allow it: C is written once and never read back here).
+template <int CPL>
+__device__ __forceinline__ void put_run(float* dst, int col, int N, const float (&out)[CPL], bool vec, bool add) {
+    if constexpr (CPL % 4 == 0) {
+        if (vec && col + CPL <= N) {
+#pragma unroll
+            for (int cc = 0; cc < CPL; cc += 4)
+                put4(dst + col + cc, f32x4{out[cc], out[cc + 1], out[cc + 2], out[cc + 3]}, add);
+            return;
+        }
+    }
+#pragma unroll
+    for (int cc = 0; cc < CPL; ++cc)
+        if (col + cc < N) put1(dst + col + cc, out[cc], add);
+}
+
+// Sum of the four waves' accumulators, in wave order, for row r = wave of every
+// group of four rows: out[c] = sum over waves of acc[c][r].  Four accumulators
+// at a time, so the LDS (16 KB) bounds no kernel's occupancy.
+template <int COUNT>
+__device__ __forceinline__ void sum_waves(const f32x4 (&acc)[COUNT], float (&out)[COUNT]) {
+    constexpr int kStage = COUNT < 4 ? COUNT : 4;
+    __shared__ float part[kWavesPerBlock][kStage * 4][kWave];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int c0 = 0; c0 < COUNT; c0 += kStage) {
+        if (c0) __syncthreads();
+#pragma unroll
+        for (int c = 0; c < kStage; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[wave][c * 4 + r][lane] = acc[c0 + c][r];
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < kStage; ++c) {
+            float v = part[0][c * 4 + wave][lane];
+#pragma unroll
+            for (int k = 1; k < kWavesPerBlock; ++k) v += part[k][c * 4 + wave][lane];
+            out[c0 + c] = v;
+        }
     }
 }
 
 // ------------------------------------------------------------ MFMA route
-template <int CPL, bool BF16, int KIND>
+template <int CPL, bool BF16, typename BRows>
 __global__ __launch_bounds__(kBlock) void tile_mfma_kernel(
     Items it, const int32_t* __restrict__ atox, const uint16_t* __restrict__ vals,
-    const uint16_t* __restrict__ Bh, int ldb, float* __restrict__ C, float* __restrict__ scratch,
-    int M, int N, int num_items, int nslices, int remap, float unscale, int vec_store) {
-    typedef typename HalfRun<CPL>::T Run;
+    const uint16_t* __restrict__ Bh, int K, int ldb, float* __restrict__ C, float* __restrict__ scratch,
+    int M, int N, int num_items, int nslices, int order, float unscale, int vec_store) {
     const int lane = threadIdx.x & (kWave - 1);
-    int64_t item_blk;
-    int slice;
-    tile_block_coords(nslices, remap, item_blk, slice);
-    const int item = __builtin_amdgcn_readfirstlane(
-        static_cast<int>(item_blk * kWavesPerBlock + (threadIdx.x >> 6)));
-    if (item >= num_items) return;
-    int w, b0, b1, slot;
-    item_range(it, item, w, b0, b1, slot);
+    WaveWork wk;
+    if (!wave_work(it, num_items, nslices, order, 4, wk)) return;
+    const int b0 = wk.b0, b1 = wk.b1;
     const int j = lane & 15;
     const int q = lane >> 4;
-    const int col = slice * (16 * CPL) + j * CPL;
-    const bool col_ok = col < ldb;  // ldb % 8 == 0 and CPL | 8: whole run in bounds
+    const int col = wk.slice * (16 * CPL) + j * CPL;
+    const bool in_row = col < ldb;  // ldb % 8 == 0 and CPL | 8: whole runs
+    const BRows rows(Bh, K, ldb, col);
     const bool a_half = (j < 8) == (q < 2);
 
     f32x4 acc[CPL];
 #pragma unroll
     for (int cc = 0; cc < CPL; ++cc) acc[cc] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // Column indices come 32 blocks (8 steps) at a time: one 16-byte load per
+    // Column keys come 32 blocks (8 steps) at a time: one 16-byte load per
     // lane (lane L: indices 4L..4L+3, half L&1 of block c0 + L/2), handed to
     // step s's lane group q (block c0 + 4s + q) from lanes 8s + 2q and
     // 8s + 2q + 1 by lane permutes, which use the LDS unit, not the address
@@ -170,9 +313,7 @@ __global__ __launch_bounds__(kBlock) void tile_mfma_kernel(
     // row, !a_half) loads the same row of block b+4+q, handed over on the odd
     // step by a lane exchange.  The pair is loaded one step ahead.
     auto load_chunk = [&](int c0) {
-        int4 v = make_int4(-1, -1, -1, -1);
-        if (c0 + (lane >> 1) < b1) v = *reinterpret_cast<const int4*>(atox + (int64_t)c0 * 8 + lane * 4);
-        return v;
+        return load_chunk4(atox, (int64_t)c0 * 8 + lane * 4, c0 + (lane >> 1) < b1);
     };
     auto load_pair = [&](int b) {  // b = first block of an even step
         const int blk = b + q + (a_half ? 0 : 4);
@@ -180,23 +321,18 @@ __global__ __launch_bounds__(kBlock) void tile_mfma_kernel(
         if (blk < b1) a = *reinterpret_cast<const u16x8*>(vals + (int64_t)blk * 64 + (j & 7) * 8);
         return a;
     };
-    int4 chunk = load_chunk(b0), chunk_next = make_int4(-1, -1, -1, -1);
+    int4 chunk, chunk_next = make_int4(-1, -1, -1, -1);
     u16x8 apair = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    if (b0 < b1) apair = load_pair(b0);
+    if (b0 < b1) {
+        chunk = chunk_keys(rows, load_chunk(b0));
+        apair = load_pair(b0);
+    }
     for (int b = b0; b < b1; b += 4) {
         const int t = (b - b0) >> 2;
         const int s = t & 7;
         if (s == 0 && b + 32 < b1) chunk_next = load_chunk(b + 32);  // one chunk ahead
-        const int l0 = 8 * s + 2 * q;
-        int cols[8];
-        cols[0] = __shfl(chunk.x, l0, kWave);
-        cols[1] = __shfl(chunk.y, l0, kWave);
-        cols[2] = __shfl(chunk.z, l0, kWave);
-        cols[3] = __shfl(chunk.w, l0, kWave);
-        cols[4] = __shfl(chunk.x, l0 + 1, kWave);
-        cols[5] = __shfl(chunk.y, l0 + 1, kWave);
-        cols[6] = __shfl(chunk.z, l0 + 1, kWave);
-        cols[7] = __shfl(chunk.w, l0 + 1, kWave);
+        int keys[8];
+        share_keys(chunk, 8 * s + 2 * q, keys);
         u16x8 a;
         if ((t & 1) == 0) {
             a = a_half ? apair : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
@@ -210,16 +346,16 @@ __global__ __launch_bounds__(kBlock) void tile_mfma_kernel(
             o[3] = __shfl_xor(mine[3], 8, kWave);
             a = a_half ? __builtin_bit_cast(u16x8, o) : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
         }
-        Run raw[8];
+        typename BRows::Run raw[8];
+        // Lanes past the row's end or the item's last block load nothing.
+        if (in_row && b + q < b1) {
+            gather8(rows, keys, raw);
+        } else {
 #pragma unroll
-        for (int v = 0; v < 8; ++v) {
-            if (cols[v] >= 0 && col_ok)
-                raw[v] = *reinterpret_cast<const Run*>(Bh + (int64_t)cols[v] * ldb + col);
-            else
-                raw[v] = Run{};
+            for (int v = 0; v < 8; ++v) raw[v] = typename BRows::Run{};
         }
         if ((t & 1) == 1 && b + 4 < b1) apair = load_pair(b + 4);
-        if (s == 7) chunk = chunk_next;
+        if (s == 7) chunk = chunk_keys(rows, chunk_next);
 #pragma unroll
         for (int cc = 0; cc < CPL; ++cc) {
             u16x8 bop;
@@ -231,39 +367,34 @@ __global__ __launch_bounds__(kBlock) void tile_mfma_kernel(
 
     // D[m][n]: lane holds rows 4*(lane>>4)+r, column n = lane & 15.  Rows m and
     // m+8 are partial sums of the same window row (block-diagonal A): lanes L
-    // and L^32 exchange them, so both halves hold the window's sums and each
-    // half stores two of its four rows (every lane stores).
+    // and L^32 exchange them.
+    const bool add = it.accumulate && wk.slot < 0;
+    float out[CPL];
+    if (wk.shared) {
+        sum_waves(acc, out);
 #pragma unroll
-    for (int cc = 0; cc < CPL; ++cc)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[cc][r] += __shfl_xor(acc[cc][r], 32, kWave);
-    // The lane's CPL columns are contiguous: 16-byte streaming stores when the
-    // rows allow it (C is written once and never read back here).
-    const bool vec = (CPL % 4 == 0) && vec_store && col + CPL <= N;
-    const bool upper = lane >= 32;  // rows 2, 3 of the lane's group of four
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int m = 4 * ((lane >> 4) & 1) + (upper ? 2 : 0) + k;
-        float out[CPL];
-#pragma unroll
-        for (int cc = 0; cc < CPL; ++cc) out[cc] = (upper ? acc[cc][2 + k] : acc[cc][k]) * unscale;  // exact
-        float* dst = item_row<KIND>(it, C, scratch, w, slot, m, M, N);
-        if (!dst) continue;
-        const bool add = it.accumulate && slot < 0;
-        if constexpr (CPL % 4 == 0) {
-            if (vec) {
-#pragma unroll
-                for (int cc = 0; cc < CPL; cc += 4)
-                    put4(dst + col + cc, f32x4{out[cc], out[cc + 1], out[cc + 2], out[cc + 3]}, add);
-                continue;
-            }
-        }
+        for (int cc = 0; cc < CPL; ++cc) out[cc] = (out[cc] + __shfl_xor(out[cc], 32, kWave)) * unscale;
+        if (lane >= 32) return;
+        float* dst = item_row(it, C, scratch, wk.w, wk.slot, 4 * (lane >> 4) + static_cast<int>(threadIdx.x >> 6), M, N);
+        if (dst) put_run<CPL>(dst, col, N, out, vec_store, add);
+    } else {
+        // Both halves then hold the window's sums and each half stores two of
+        // its four rows (every lane stores).
 #pragma unroll
         for (int cc = 0; cc < CPL; ++cc)
-            if (col + cc < N) put1(dst + col + cc, out[cc], add);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[cc][r] += __shfl_xor(acc[cc][r], 32, kWave);
+        const bool upper = lane >= 32;  // rows 2, 3 of the lane's group of four
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int m = 4 * ((lane >> 4) & 1) + (upper ? 2 : 0) + k;
+#pragma unroll
+            for (int cc = 0; cc < CPL; ++cc) out[cc] = (upper ? acc[cc][2 + k] : acc[cc][k]) * unscale;  // exact
+            float* dst = item_row(it, C, scratch, wk.w, wk.slot, m, M, N);
+            if (dst) put_run<CPL>(dst, col, N, out, vec_store, add);
+        }
     }
 }
-
 
 // ------------------------------------------------- MFMA route, tall windows
 // Windows of H = 16*RG rows; a block is 32 vectors (one MFMA K) with values
@@ -272,115 +403,92 @@ __global__ __launch_bounds__(kBlock) void tile_mfma_kernel(
 // row group), so a B row shared by several of the H rows is gathered once.
 // Per step: one index load (lane pairs exchange halves), 8 B-row gathers,
 // RG A loads; no block-diagonal padding.
-template <int CPL, bool BF16, int KIND, int RG>
+template <int CPL, bool BF16, int RG, typename BRows>
 __global__ __launch_bounds__(kBlock) void tile_mfma_tall_kernel(
     Items it, const int32_t* __restrict__ atox, const uint16_t* __restrict__ vals,
-    const uint16_t* __restrict__ Bh, int ldb, float* __restrict__ C, float* __restrict__ scratch,
+    const uint16_t* __restrict__ Bh, int K, int ldb, float* __restrict__ C, float* __restrict__ scratch,
     int M, int N, int num_items, int nslices, int order, float unscale, int vec_store) {
-    typedef typename HalfRun<CPL>::T Run;
     constexpr int H = 16 * RG;
     constexpr int BV = H * 32;  // values per block
     const int lane = threadIdx.x & (kWave - 1);
-    int64_t item_blk;
-    int slice;
-    tile_block_coords(nslices, order, item_blk, slice);
-    const int item = __builtin_amdgcn_readfirstlane(
-        static_cast<int>(item_blk * kWavesPerBlock + (threadIdx.x >> 6)));
-    if (item >= num_items) return;
-    int w, b0, b1, slot;
-    item_range(it, item, w, b0, b1, slot);
+    WaveWork wk;
+    if (!wave_work(it, num_items, nslices, order, 1, wk)) return;
+    const int b0 = wk.b0, b1 = wk.b1;
     const int j = lane & 15;
     const int q = lane >> 4;
-    const int col = slice * (16 * CPL) + j * CPL;
-    const bool col_ok = col < ldb;
+    const int col = wk.slice * (16 * CPL) + j * CPL;
+    // Lanes past the row's end gather its last run again and store nothing.
+    const BRows rows(Bh, K, ldb, min(col, ldb - CPL));
 
-    f32x4 acc[RG][CPL];
+    f32x4 acc[RG * CPL];
 #pragma unroll
-    for (int g = 0; g < RG; ++g)
-#pragma unroll
-        for (int cc = 0; cc < CPL; ++cc) acc[g][cc] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < RG * CPL; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // Column indices come 8 blocks at a time: one 16-byte load per lane
+    // Column keys come 8 blocks at a time: one 16-byte load per lane
     // covers the 256 indices of blocks [c0, c0 + 8) (lane L: indices 4L..4L+3),
     // and step b takes its 8 from lanes 8s + 2q and 8s + 2q + 1 (s = b - c0)
     // by lane permutes, which use the LDS unit, not the address unit.
     auto load_chunk = [&](int c0) {
-        int4 v = make_int4(-1, -1, -1, -1);
-        if (c0 + (lane >> 3) < b1) v = *reinterpret_cast<const int4*>(atox + (int64_t)c0 * 32 + lane * 4);
-        return v;
-    };
-    auto cols_of = [&](const int4& chunk, int s, int (&cols)[8]) {
-        const int l0 = 8 * s + 2 * q;
-        cols[0] = __shfl(chunk.x, l0, kWave);
-        cols[1] = __shfl(chunk.y, l0, kWave);
-        cols[2] = __shfl(chunk.z, l0, kWave);
-        cols[3] = __shfl(chunk.w, l0, kWave);
-        cols[4] = __shfl(chunk.x, l0 + 1, kWave);
-        cols[5] = __shfl(chunk.y, l0 + 1, kWave);
-        cols[6] = __shfl(chunk.z, l0 + 1, kWave);
-        cols[7] = __shfl(chunk.w, l0 + 1, kWave);
+        return load_chunk4(atox, (int64_t)c0 * 32 + lane * 4, c0 + (lane >> 3) < b1);
     };
     auto load_a = [&](int b, u16x8 (&a)[RG]) {
 #pragma unroll
         for (int g = 0; g < RG; ++g)
             a[g] = *reinterpret_cast<const u16x8*>(vals + (int64_t)b * BV + ((g * 4 + q) * 16 + j) * 8);
     };
-    int4 chunk = load_chunk(b0), chunk_next = make_int4(-1, -1, -1, -1);
+    int4 chunk, chunk_next = make_int4(-1, -1, -1, -1);
     u16x8 a_next[RG];
-    if (b0 < b1) load_a(b0, a_next);
+    if (b0 < b1) {
+        chunk = chunk_keys(rows, load_chunk(b0));
+        load_a(b0, a_next);
+    }
     for (int b = b0; b < b1; ++b) {
         const int s = (b - b0) & 7;
         if (s == 0 && b + 8 < b1) chunk_next = load_chunk(b + 8);  // one chunk ahead
-        int cols[8];
-        cols_of(chunk, s, cols);
+        int keys[8];
+        share_keys(chunk, 8 * s + 2 * q, keys);
         u16x8 a[RG];
 #pragma unroll
         for (int g = 0; g < RG; ++g) a[g] = a_next[g];
-        Run raw[8];
-#pragma unroll
-        for (int v = 0; v < 8; ++v) {
-            if (cols[v] >= 0 && col_ok)
-                raw[v] = *reinterpret_cast<const Run*>(Bh + (int64_t)cols[v] * ldb + col);
-            else
-                raw[v] = Run{};
-        }
+        typename BRows::Run raw[8];
+        gather8(rows, keys, raw);
         if (b + 1 < b1) load_a(b + 1, a_next);
-        if (s == 7) chunk = chunk_next;
+        if (s == 7) chunk = chunk_keys(rows, chunk_next);
 #pragma unroll
         for (int cc = 0; cc < CPL; ++cc) {
             u16x8 bop;
 #pragma unroll
             for (int v = 0; v < 8; ++v) bop[v] = run_elem<CPL>(raw[v], cc);
 #pragma unroll
-            for (int g = 0; g < RG; ++g) acc[g][cc] = mfma32<BF16>(a[g], bop, acc[g][cc]);
+            for (int g = 0; g < RG; ++g) acc[g * CPL + cc] = mfma32<BF16>(a[g], bop, acc[g * CPL + cc]);
         }
     }
 
     // D of row group g: lane holds rows 16g + 4q + r, column j's CPL outputs.
-    const bool vec = (CPL % 4 == 0) && vec_store && col + CPL <= N;
+    const bool add = it.accumulate && wk.slot < 0;
+    auto put = [&](int g, int r, const float (&out)[CPL]) {
+        float* dst = item_row<H>(it, C, scratch, wk.w, wk.slot, 16 * g + 4 * q + r, M, N);
+        if (dst) put_run<CPL>(dst, col, N, out, vec_store, add);
+    };
+    float out[CPL];
+    if (wk.shared) {
+        float sums[RG * CPL];
+        sum_waves(acc, sums);
 #pragma unroll
-    for (int g = 0; g < RG; ++g) {
+        for (int g = 0; g < RG; ++g) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int m = 16 * g + 4 * q + r;
-            float* dst = item_row<KIND, H>(it, C, scratch, w, slot, m, M, N);
-            if (!dst) continue;
-            float out[CPL];
-#pragma unroll
-            for (int cc = 0; cc < CPL; ++cc) out[cc] = acc[g][cc][r] * unscale;  // exact: power of two
-            const bool add = it.accumulate && slot < 0;
-            if constexpr (CPL % 4 == 0) {
-                if (vec) {
-#pragma unroll
-                    for (int cc = 0; cc < CPL; cc += 4)
-                        put4(dst + col + cc, f32x4{out[cc], out[cc + 1], out[cc + 2], out[cc + 3]}, add);
-                    continue;
-                }
-            }
-#pragma unroll
-            for (int cc = 0; cc < CPL; ++cc)
-                if (col + cc < N) put1(dst + col + cc, out[cc], add);
+            for (int cc = 0; cc < CPL; ++cc) out[cc] = sums[g * CPL + cc] * unscale;
+            put(g, threadIdx.x >> 6, out);
         }
+    } else {
+#pragma unroll
+        for (int g = 0; g < RG; ++g)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+#pragma unroll
+                for (int cc = 0; cc < CPL; ++cc) out[cc] = acc[g * CPL + cc][r] * unscale;  // exact: power of two
+                put(g, r, out);
+            }
     }
 }
 
@@ -403,26 +511,21 @@ __device__ __forceinline__ f32x16 mfma3232(u16x8 a, u16x8 b, f32x16 c) {
                                                       __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
-template <bool BF16, int KIND>
+template <bool BF16, typename BRows>
 __global__ __launch_bounds__(kBlock, 2) void tile_mfma_tall32_kernel(
     Items it, const int32_t* __restrict__ atox, const uint16_t* __restrict__ vals,
-    const uint16_t* __restrict__ Bh, int ldb, float* __restrict__ C, float* __restrict__ scratch,
+    const uint16_t* __restrict__ Bh, int K, int ldb, float* __restrict__ C, float* __restrict__ scratch,
     int M, int N, int num_items, int nslices, int order, float unscale, int vec_store) {
     constexpr int H = 32;
     constexpr int BV = H * 32;  // values per block
     const int lane = threadIdx.x & (kWave - 1);
-    int64_t item_blk;
-    int slice;
-    tile_block_coords(nslices, order, item_blk, slice);
-    const int item = __builtin_amdgcn_readfirstlane(
-        static_cast<int>(item_blk * kWavesPerBlock + (threadIdx.x >> 6)));
-    if (item >= num_items) return;
-    int w, b0, b1, slot;
-    item_range(it, item, w, b0, b1, slot);
+    WaveWork wk;
+    if (!wave_work(it, num_items, nslices, order, 1, wk)) return;
+    const int b0 = wk.b0, b1 = wk.b1;
     const int j = lane & 31;
     const int q = lane >> 5;
-    const int col = slice * 256 + j * 8;
-    const bool col_ok = col < ldb;
+    const int col = wk.slice * 256 + j * 8;
+    const BRows rows(Bh, K, ldb, min(col, ldb - 8));
     // A operand of row j, k-group q4: offset in the [2][4][16][8] block layout.
     const int a_row = ((j >> 4) * 4) * 16 + (j & 15);
 
@@ -435,36 +538,20 @@ __global__ __launch_bounds__(kBlock, 2) void tile_mfma_tall32_kernel(
     // Column indices: one 16-byte load per lane covers blocks [c0, c0 + 8);
     // block s, k-group q4 sits in lanes 8s + 2q4 and 8s + 2q4 + 1.
     auto load_chunk = [&](int c0) {
-        int4 v = make_int4(-1, -1, -1, -1);
-        if (c0 + (lane >> 3) < b1) v = *reinterpret_cast<const int4*>(atox + (int64_t)c0 * 32 + lane * 4);
-        return v;
+        return load_chunk4(atox, (int64_t)c0 * 32 + lane * 4, c0 + (lane >> 3) < b1);
     };
-    int4 chunk = load_chunk(b0), chunk_next = make_int4(-1, -1, -1, -1);
+    int4 chunk = chunk_keys(rows, load_chunk(b0)), chunk_next = make_int4(-1, -1, -1, -1);
     for (int b = b0; b < b1; ++b) {
         const int s = (b - b0) & 7;
         if (s == 0 && b + 8 < b1) chunk_next = load_chunk(b + 8);
 #pragma unroll 1
         for (int h = 0; h < 2; ++h) {
             const int q4 = 2 * h + q;
-            int cols[8];
-            const int l0 = 8 * s + 2 * q4;
-            cols[0] = __shfl(chunk.x, l0, kWave);
-            cols[1] = __shfl(chunk.y, l0, kWave);
-            cols[2] = __shfl(chunk.z, l0, kWave);
-            cols[3] = __shfl(chunk.w, l0, kWave);
-            cols[4] = __shfl(chunk.x, l0 + 1, kWave);
-            cols[5] = __shfl(chunk.y, l0 + 1, kWave);
-            cols[6] = __shfl(chunk.z, l0 + 1, kWave);
-            cols[7] = __shfl(chunk.w, l0 + 1, kWave);
+            int keys[8];
+            share_keys(chunk, 8 * s + 2 * q4, keys);
             const u16x8 a = *reinterpret_cast<const u16x8*>(vals + (int64_t)b * BV + (a_row + q4 * 16) * 8);
             u16x8 raw[8];
-#pragma unroll
-            for (int v = 0; v < 8; ++v) {
-                if (cols[v] >= 0 && col_ok)
-                    raw[v] = *reinterpret_cast<const u16x8*>(Bh + (int64_t)cols[v] * ldb + col);
-                else
-                    raw[v] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            }
+            gather8(rows, keys, raw);
 #pragma unroll
             for (int cc = 0; cc < 8; ++cc) {
                 u16x8 bop;
@@ -473,27 +560,18 @@ __global__ __launch_bounds__(kBlock, 2) void tile_mfma_tall32_kernel(
                 acc[cc] = mfma3232<BF16>(a, bop, acc[cc]);
             }
         }
-        if (s == 7) chunk = chunk_next;
+        if (s == 7) chunk = chunk_keys(rows, chunk_next);
     }
 
-    const bool vec = vec_store && col + 8 <= N;
+    const bool add = it.accumulate && wk.slot < 0;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int m = 8 * (i >> 2) + 4 * q + (i & 3);
-        float* dst = item_row<KIND, H>(it, C, scratch, w, slot, m, M, N);
-        if (!dst) continue;
+        float* dst = item_row<H>(it, C, scratch, wk.w, wk.slot, m, M, N);
         float out[8];
 #pragma unroll
         for (int cc = 0; cc < 8; ++cc) out[cc] = acc[cc][i] * unscale;  // exact: power of two
-        const bool add = it.accumulate && slot < 0;
-        if (vec) {
-            put4(dst + col, f32x4{out[0], out[1], out[2], out[3]}, add);
-            put4(dst + col + 4, f32x4{out[4], out[5], out[6], out[7]}, add);
-        } else {
-#pragma unroll
-            for (int cc = 0; cc < 8; ++cc)
-                if (col + cc < N) put1(dst + col + cc, out[cc], add);
-        }
+        if (dst) put_run<8>(dst, col, N, out, vec_store, add);
     }
 }
 
@@ -616,11 +694,11 @@ int tile_slice_major(int nslices, bool remapped) {
 
 // One launch's share of a plan: all of it, or one column partition.
 struct Part {
-    int item_base, num_items, cell_base, accumulate, split_base, num_splits;
+    int item_base, num_items, cell_base, accumulate, split_base, num_splits, num_long;
 };
 
 Part whole_plan(const ra_tile_plan* p) {
-    return Part{0, p->num_items, 0, 0, 0, p->info.num_split_windows};
+    return Part{0, p->num_items, 0, 0, 0, p->info.num_split_windows, p->part_long[0]};
 }
 
 Items plan_items(const ra_tile_plan* p, const Part& part) {
@@ -628,87 +706,111 @@ Items plan_items(const ra_tile_plan* p, const Part& part) {
     it.item_base = part.item_base;
     it.cell_base = part.cell_base;
     it.accumulate = part.accumulate;
+    it.order = p->has_long ? p->item_order.get<int32_t>() : nullptr;
     it.block_offsets = p->block_offsets.get<int32_t>();
     it.seg_window = p->seg_window.get<int32_t>();
     it.seg_bbegin = p->seg_bbegin.get<int32_t>();
     it.seg_bend = p->seg_bend.get<int32_t>();
     it.seg_slot = p->seg_slot.get<int32_t>();
-    it.win_rows = p->win_rows.get<int32_t>();
+    it.win_rows = p->info.kind == RA_TILE_COMMUNITY_TC ? p->win_rows.get<int32_t>() : nullptr;
     return it;
 }
 
-template <int KIND>
-ra_status launch_mfma_kind(const ra_tile_plan* p, const Part& part, const uint16_t* Bh, int ldb, bool bf16,
-                           float* C, float* scratch, int N, hipStream_t st) {
-    const int M = p->info.M;
-    const Items it = plan_items(p, part);
-    int cpl = N <= 16 ? 1 : N <= 32 ? 2 : N <= 64 ? 4 : 8;
-    cpl = std::min(cpl, tile_max_cpl());
-    const int nslices = (N + 16 * cpl - 1) / (16 * cpl);
-    const int remap = (KIND == RA_TILE_COMMUNITY_TC ? 0 : tile_remap()) | (tile_slice_major(nslices, KIND != RA_TILE_COMMUNITY_TC && tile_remap()) ? 2 : 0);
-    const float unscale = std::ldexp(1.0f, -p->info.value_scale_log2);
-    dim3 grid(static_cast<unsigned>(((int64_t)part.num_items + kWavesPerBlock - 1) / kWavesPerBlock * nslices));
-    const int vec_store = (N % 4 == 0) && ra::aligned16(C) && (!scratch || ra::aligned16(scratch));
-#define RA_MFMA_CASE(c)                                                                            \
-    if (cpl == c) {                                                                                \
-        if (bf16)                                                                                  \
-            tile_mfma_kernel<c, true, KIND><<<grid, kBlock, 0, st>>>(it, p->atox.get<int32_t>(),    \
-                p->vals.get<uint16_t>(), Bh, ldb, C, scratch, M, N, part.num_items, nslices, remap, unscale, vec_store); \
-        else                                                                                       \
-            tile_mfma_kernel<c, false, KIND><<<grid, kBlock, 0, st>>>(it, p->atox.get<int32_t>(),   \
-                p->vals.get<uint16_t>(), Bh, ldb, C, scratch, M, N, part.num_items, nslices, remap, unscale, vec_store); \
-    }
-    RA_MFMA_CASE(1)
-    RA_MFMA_CASE(2)
-    RA_MFMA_CASE(4)
-    RA_MFMA_CASE(8)
-#undef RA_MFMA_CASE
-    RA_LAUNCH_CHECK("tile_mfma_kernel");
-    return RA_OK;
+// How one launch runs: columns per lane, the grid and the scheduling order.
+struct TileLaunch {
+    Items items;
+    int cpl, nslices, order, lds;
+    dim3 grid;
+    int vec_store;
+    float unscale;
+};
+
+// Bytes of B that a launch gathers (an even share of the plan's blocks).
+double gathered_bytes(const ra_tile_plan* p, int N) {
+    const int vb = p->info.rows_per_window == ra::kTileWindow ? ra::kTileVec : 32;
+    return 2.0 * N * vb * p->info.num_blocks / std::max(p->info.col_parts, 1);
+}
+constexpr double kGatherBound = 2.0 * (1u << 30);
+
+// Items of one launch that a whole workgroup shares.
+// All of them where the launch leaves much of the chip idle (fewer than 4096
+// waves; 1024 of tall windows, which hold more registers) and a quarter is worth
+// a wave: 15,000 rows of degree 30 at N = 64 (1.9e3 items of 7.5 steps) 17.9 -> 16.3
+// us, 30,000 of 200 at N = 128 (3.8e3 of 50) 87 -> 79, a community graph of 8,000
+// rows at N = 128 (250 tall items) 18.4 -> 9.0.  With shorter items it loses (10,000
+// rows of 22 at N = 176, 5.5 steps: 17.0 -> 19.4), and with more tall ones (64,000
+// rows: 43.6 -> 55.6).
+// Otherwise the long ones, whose chains of gathers (128 steps of ~0.6 us in a
+// window of 512 blocks) outlast the rest of a small launch: 50,000 rows of 80 at
+// N = 128 91 -> 84 us, 20,000 of 60 at N = 64 42 -> 21.  Where the gathered bytes
+// take longer than any chain (2 GiB, ~250 us) it only spreads the columns that
+// are gathered at a time: 100,000 rows of 60 at N = 256 33 -> 31 % L2 hits, 371
+// -> 387 us.
+int shared_items(const ra_tile_plan* p, const Part& part, int N, int nslices) {
+    const bool tall = p->info.rows_per_window != ra::kTileWindow;
+    const int64_t waves = (int64_t)part.num_items * nslices;
+    const double steps = static_cast<double>(p->info.num_blocks) / std::max(p->num_items, 1) / (tall ? 1 : 4);
+    if (waves < (tall ? 1024 : 4096) && steps >= (tall ? 4 : 7)) return part.num_items;
+    return gathered_bytes(p, N) < kGatherBound ? part.num_long : 0;
 }
 
-ra_status launch_merge(const ra_tile_plan* p, const Part& part, float* C, int N, hipStream_t st) {
-    if (part.num_splits == 0) return RA_OK;
-    const int H = p->info.rows_per_window;
-    dim3 grid(part.num_splits,
-              static_cast<unsigned>(std::min<int64_t>(((int64_t)H * N + kBlock - 1) / kBlock, 65535)));
-    const int32_t* wr = p->info.kind == RA_TILE_COMMUNITY_TC ? p->win_rows.get<int32_t>() : nullptr;
-    tile_merge_kernel<<<grid, kBlock, 0, st>>>(p->split_windows.get<int32_t>() + part.split_base,
-                                               p->split_offsets.get<int32_t>() + part.split_base, wr,
-                                               p->scratch.get<float>(), C, p->info.M, N, H, part.cell_base,
-                                               part.accumulate);
-    RA_LAUNCH_CHECK("tile_merge_kernel");
-    return RA_OK;
+// LDS that holds a launch to 3 workgroups per CU.  Windows in flight together
+// sweep the columns from left to right side by side; in a gather-bound launch
+// without column partitions fewer of them keep closer together: 100,000 rows of
+// 60 at N = 256 32.5 -> 33.8 % L2 hits, 372 -> 360 us, 50,000 of 80 at N = 512 355
+// -> 341, 500,000 of 16 at N = 256 769 -> 760.  Partitioned plans (8,890 -> 8,940 us
+// on 250,000 rows of 500 at N = 512) and shorter launches (44.8 -> 49.8) lose.
+constexpr int kFewerWaves = 53000 - 16384;
+int tile_lds(const ra_tile_plan* p, int N) {
+    return p->info.rows_per_window == ra::kTileWindow && p->info.col_parts <= 1 &&
+                   gathered_bytes(p, N) >= kGatherBound
+               ? kFewerWaves : 0;
 }
 
-template <int KIND, int RG>
-ra_status launch_mfma_tall(const ra_tile_plan* p, const Part& part, const uint16_t* Bh, int ldb, bool bf16,
-                           float* C, float* scratch, int N, hipStream_t st) {
-    const int M = p->info.M;
-    const Items it = plan_items(p, part);
-    int cpl = N <= 16 ? 1 : N <= 32 ? 2 : N <= 64 ? 4 : 8;
-    cpl = std::min(cpl, tile_max_cpl());
-    const int nslices = (N + 16 * cpl - 1) / (16 * cpl);
-    const int order = (KIND == RA_TILE_COMMUNITY_TC ? 0 : tile_remap()) | (tile_slice_major(nslices, KIND != RA_TILE_COMMUNITY_TC && tile_remap()) ? 2 : 0);
-    const float unscale = std::ldexp(1.0f, -p->info.value_scale_log2);
-    dim3 grid(static_cast<unsigned>(((int64_t)part.num_items + kWavesPerBlock - 1) / kWavesPerBlock * nslices));
-    const int vec_store = (N % 4 == 0) && ra::aligned16(C) && (!scratch || ra::aligned16(scratch));
-#define RA_TALL_CASE(c)                                                                                  \
-    if (cpl == c) {                                                                                      \
-        if (bf16)                                                                                        \
-            tile_mfma_tall_kernel<c, true, KIND, RG><<<grid, kBlock, 0, st>>>(it, p->atox.get<int32_t>(), \
-                p->vals.get<uint16_t>(), Bh, ldb, C, scratch, M, N, part.num_items, nslices, order, unscale, vec_store); \
-        else                                                                                             \
-            tile_mfma_tall_kernel<c, false, KIND, RG><<<grid, kBlock, 0, st>>>(it, p->atox.get<int32_t>(), \
-                p->vals.get<uint16_t>(), Bh, ldb, C, scratch, M, N, part.num_items, nslices, order, unscale, vec_store); \
-    }
-    RA_TALL_CASE(1)
-    RA_TALL_CASE(2)
-    RA_TALL_CASE(4)
-    RA_TALL_CASE(8)
-#undef RA_TALL_CASE
-    RA_LAUNCH_CHECK("tile_mfma_tall_kernel");
-    return RA_OK;
+TileLaunch tile_launch(const ra_tile_plan* p, const Part& part, const float* C, const float* scratch, int N,
+                       bool wide) {
+    TileLaunch l{};
+    l.cpl = std::min(N <= 16 ? 1 : N <= 32 ? 2 : N <= 64 ? 4 : 8, tile_max_cpl());
+    const int slice_cols = wide ? 256 : 16 * l.cpl;
+    l.nslices = (N + slice_cols - 1) / slice_cols;
+    const bool remap = p->info.kind != RA_TILE_COMMUNITY_TC && tile_remap();
+    l.order = (remap ? 1 : 0) | (tile_slice_major(l.nslices, remap) ? 2 : 0);
+    l.items = plan_items(p, part);
+    l.items.num_long = wide ? 0 : shared_items(p, part, N, l.nslices);
+    l.items.order = l.items.num_long == part.num_long ? l.items.order : nullptr;
+    const int64_t groups =
+        l.items.num_long + ((int64_t)part.num_items - l.items.num_long + kWavesPerBlock - 1) / kWavesPerBlock;
+    l.grid = dim3(static_cast<unsigned>(groups * l.nslices));
+    l.lds = tile_lds(p, N);
+    l.vec_store = (N % 4 == 0) && ra::aligned16(C) && (!scratch || ra::aligned16(scratch));
+    l.unscale = std::ldexp(1.0f, -p->info.value_scale_log2);
+    return l;
+}
+
+// B of K rows fits HalfBuffer: the offset of row -1 lies past its end.
+bool half_buffer_fits(int64_t K, int64_t ldb) { return (K + 1) * ldb * 2 <= int64_t{0xFFFFFFFF}; }
+
+#define RA_TILE_ARGS                                                                                       \
+    l.items, p->atox.get<int32_t>(), p->vals.get<uint16_t>(), Bh, p->info.K, ldb, C, scratch, \
+        p->info.M, N, part.num_items, l.nslices, l.order, l.unscale, l.vec_store
+
+template <int CPL, bool BF16, template <int> class BRows>
+void launch_tile(const ra_tile_plan* p, const Part& part, const TileLaunch& l, const uint16_t* Bh, int ldb, float* C,
+                 float* scratch, int N, hipStream_t st) {
+    const int h = p->info.rows_per_window;
+    if (h == 32) tile_mfma_tall_kernel<CPL, BF16, 2, BRows<CPL>><<<l.grid, kBlock, 0, st>>>(RA_TILE_ARGS);
+    else if (h == 16) tile_mfma_tall_kernel<CPL, BF16, 1, BRows<CPL>><<<l.grid, kBlock, 0, st>>>(RA_TILE_ARGS);
+    else tile_mfma_kernel<CPL, BF16, BRows<CPL>><<<l.grid, kBlock, l.lds, st>>>(RA_TILE_ARGS);
+}
+
+template <bool BF16, template <int> class BRows>
+void launch_cpl(const ra_tile_plan* p, const Part& part, const TileLaunch& l, const uint16_t* Bh, int ldb, float* C,
+                float* scratch, int N, hipStream_t st) {
+    auto f = l.cpl == 1   ? launch_tile<1, BF16, BRows>
+             : l.cpl == 2 ? launch_tile<2, BF16, BRows>
+             : l.cpl == 4 ? launch_tile<4, BF16, BRows>
+                          : launch_tile<8, BF16, BRows>;
+    f(p, part, l, Bh, ldb, C, scratch, N, st);
 }
 
 // 32-row windows run on the 32x32x16 MFMA kernel at N >= 512 (C3 N=512:
@@ -724,40 +826,38 @@ bool tile_use_mfma32(int N) {
     return N >= 512;
 }
 
-template <int KIND>
-ra_status launch_mfma_tall32(const ra_tile_plan* p, const Part& part, const uint16_t* Bh, int ldb, bool bf16,
-                             float* C, float* scratch, int N, hipStream_t st) {
-    const int M = p->info.M;
-    const Items it = plan_items(p, part);
-    const int nslices = (N + 255) / 256;
-    const int order = (KIND == RA_TILE_COMMUNITY_TC ? 0 : tile_remap()) |
-                      (tile_slice_major(nslices, KIND != RA_TILE_COMMUNITY_TC && tile_remap()) ? 2 : 0);
-    const float unscale = std::ldexp(1.0f, -p->info.value_scale_log2);
-    dim3 grid(static_cast<unsigned>(((int64_t)part.num_items + kWavesPerBlock - 1) / kWavesPerBlock * nslices));
-    const int vec_store = (N % 4 == 0) && ra::aligned16(C) && (!scratch || ra::aligned16(scratch));
-    if (bf16)
-        tile_mfma_tall32_kernel<true, KIND><<<grid, kBlock, 0, st>>>(it, p->atox.get<int32_t>(),
-            p->vals.get<uint16_t>(), Bh, ldb, C, scratch, M, N, part.num_items, nslices, order, unscale, vec_store);
-    else
-        tile_mfma_tall32_kernel<false, KIND><<<grid, kBlock, 0, st>>>(it, p->atox.get<int32_t>(),
-            p->vals.get<uint16_t>(), Bh, ldb, C, scratch, M, N, part.num_items, nslices, order, unscale, vec_store);
-    RA_LAUNCH_CHECK("tile_mfma_tall32_kernel");
+template <bool BF16>
+ra_status launch_part(const ra_tile_plan* p, const Part& part, const uint16_t* Bh, int ldb, float* C, float* scratch,
+                      int N, hipStream_t st) {
+    if (part.num_items == 0) return RA_OK;
+    const bool wide = p->info.rows_per_window == 32 && tile_use_mfma32(N);
+    const TileLaunch l = tile_launch(p, part, C, scratch, N, wide);
+    // Wide rows of a partitioned plan gather no faster without the branches, and
+    // the branches keep the windows in step: 250,000 rows of 500 at N = 512 8,880 us
+    // through the buffer, 8,840 through pointers (N = 128, one slice: 690 and 745 on
+    // 150,000 rows of 200).
+    const bool buf = half_buffer_fits(p->info.K, ldb) &&
+                     !(p->info.col_parts > 1 && l.nslices > 1 && p->info.rows_per_window == ra::kTileWindow);
+    if (!wide) (buf ? launch_cpl<BF16, HalfBuffer> : launch_cpl<BF16, HalfPointer>)(p, part, l, Bh, ldb, C, scratch, N, st);
+    else if (buf) tile_mfma_tall32_kernel<BF16, HalfBuffer<8>><<<l.grid, kBlock, 0, st>>>(RA_TILE_ARGS);
+    else tile_mfma_tall32_kernel<BF16, HalfPointer<8>><<<l.grid, kBlock, 0, st>>>(RA_TILE_ARGS);
+    RA_LAUNCH_CHECK("tile_mfma_kernel");
     return RA_OK;
 }
+#undef RA_TILE_ARGS
 
-template <int KIND>
-ra_status launch_kind(const ra_tile_plan* p, const Part& part, const uint16_t* Bh, int ldb, bool bf16, float* C,
-                      float* scratch, int N, hipStream_t st) {
-    if (part.num_items == 0) return RA_OK;
-    switch (p->info.rows_per_window) {
-        case 16:
-            return launch_mfma_tall<KIND, 1>(p, part, Bh, ldb, bf16, C, scratch, N, st);
-        case 32:
-            if (tile_use_mfma32(N)) return launch_mfma_tall32<KIND>(p, part, Bh, ldb, bf16, C, scratch, N, st);
-            return launch_mfma_tall<KIND, 2>(p, part, Bh, ldb, bf16, C, scratch, N, st);
-        default:
-            return launch_mfma_kind<KIND>(p, part, Bh, ldb, bf16, C, scratch, N, st);
-    }
+ra_status launch_merge(const ra_tile_plan* p, const Part& part, float* C, int N, hipStream_t st) {
+    if (part.num_splits == 0) return RA_OK;
+    const int H = p->info.rows_per_window;
+    dim3 grid(part.num_splits,
+              static_cast<unsigned>(std::min<int64_t>(((int64_t)H * N + kBlock - 1) / kBlock, 65535)));
+    const int32_t* wr = p->info.kind == RA_TILE_COMMUNITY_TC ? p->win_rows.get<int32_t>() : nullptr;
+    tile_merge_kernel<<<grid, kBlock, 0, st>>>(p->split_windows.get<int32_t>() + part.split_base,
+                                               p->split_offsets.get<int32_t>() + part.split_base, wr,
+                                               p->scratch.get<float>(), C, p->info.M, N, H, part.cell_base,
+                                               part.accumulate);
+    RA_LAUNCH_CHECK("tile_merge_kernel");
+    return RA_OK;
 }
 
 // FP16/BF16 MFMA route over 16-bit B (converted, or passed in by the caller).
@@ -774,18 +874,9 @@ ra_status run_common(ra_tile_plan* p, const uint16_t* Bh, int ldb, bool bf16, fl
         const Part part = P == 1 ? whole_plan(p)
                                  : Part{p->part_items[q], p->part_items[q + 1] - p->part_items[q],
                                         q * p->info.num_windows, q > 0 ? 1 : 0, p->part_splits[q],
-                                        p->part_splits[q + 1] - p->part_splits[q]};
-        switch (p->info.kind) {
-            case RA_TILE_TC_DIRECT:
-                RA_TRY(launch_kind<RA_TILE_TC_DIRECT>(p, part, Bh, ldb, bf16, C, scratch, N, st));
-                break;
-            case RA_TILE_COMMUNITY_TC:
-                RA_TRY(launch_kind<RA_TILE_COMMUNITY_TC>(p, part, Bh, ldb, bf16, C, scratch, N, st));
-                break;
-            default:
-                RA_TRY(launch_kind<RA_TILE_SEGMENT_HYBRID>(p, part, Bh, ldb, bf16, C, scratch, N, st));
-                break;
-        }
+                                        p->part_splits[q + 1] - p->part_splits[q], p->part_long[q]};
+        RA_TRY(bf16 ? launch_part<true>(p, part, Bh, ldb, C, scratch, N, st)
+                    : launch_part<false>(p, part, Bh, ldb, C, scratch, N, st));
         RA_TRY(launch_merge(p, part, C, N, st));
     }
     return RA_OK;
@@ -833,6 +924,15 @@ ra_status ra_tile_plan_create(int32_t kind, const int32_t* h_rowptr, const int32
             (s = p->split_windows.upload(host.split_windows)) == RA_OK &&
             (s = p->split_offsets.upload(host.split_offsets)) == RA_OK) {
             p->num_items = p->info.num_segments;
+            std::vector<int32_t> order;
+            for (int pass = 0; pass < 2; ++pass)
+                for (int32_t i = 0; i < p->num_items; ++i)
+                    if ((host.seg_bend[i] - host.seg_bbegin[i] > ra::kTileLongBlocks) == (pass == 0)) {
+                        order.push_back(i);
+                        p->part_long[0] += pass == 0;
+                    }
+            p->has_long = p->part_long[0] > 0;
+            s = p->item_order.upload(order);
         }
     }
     if (s != RA_OK) {
