@@ -577,47 +577,78 @@ __global__ __launch_bounds__(kBlock, 2) void tile_mfma_tall32_kernel(
 
 // ------------------------------------------------ SEGMENT_HYBRID merge
 // C[w*8+m][n] = ((slot0 + slot1) + ...) in ascending slot order
-// (tc/ra_segment_hybrid.cu:198-221).
+// (tc/ra_segment_hybrid.cu:198-221).  A thread owns one column of one window
+// row and loads kDeep slots at a time, so a long window's chain is its additions
+// and not a memory latency per slot.
 __global__ __launch_bounds__(kBlock) void tile_merge_kernel(
     const int32_t* __restrict__ split_windows, const int32_t* __restrict__ split_offsets,
     const int32_t* __restrict__ win_rows, const float* __restrict__ scratch, float* __restrict__ C,
     int M, int N, int H, int cell_base, int accumulate) {
+    constexpr int kDeep = 8;
     const int sw = blockIdx.x;
     const int o0 = split_offsets[sw], o1 = split_offsets[sw + 1];
+    const int64_t window = split_windows[sw] - cell_base;
+    const uint32_t count = static_cast<uint32_t>(H) * N;
     // grid.y is capped by the launch; stride over the window's H*N elements.
-    for (int64_t e = (int64_t)blockIdx.y * kBlock + threadIdx.x; e < (int64_t)H * N;
-         e += (int64_t)gridDim.y * kBlock) {
-        const int m = static_cast<int>(e / N);
-        const int n = static_cast<int>(e - (int64_t)m * N);
-        const int64_t slot_row = (int64_t)(split_windows[sw] - cell_base) * H + m;
+    for (uint32_t e = blockIdx.y * kBlock + threadIdx.x; e < count; e += gridDim.y * kBlock) {
+        const uint32_t m = e / static_cast<uint32_t>(N);
+        const int64_t slot_row = window * H + m;
         const int row = win_rows ? win_rows[slot_row] : static_cast<int>(slot_row);
         if (row < 0 || row >= M) continue;
-        float acc = scratch[((int64_t)o0 * H + m) * N + n];
-        for (int o = o0 + 1; o < o1; ++o) acc += scratch[((int64_t)o * H + m) * N + n];
-        if (accumulate) acc = C[(int64_t)row * N + n] + acc;
-        C[(int64_t)row * N + n] = acc;
+        const float* part = scratch + e;
+        float acc = part[(int64_t)o0 * count];
+        int o = o0 + 1;
+        for (; o + kDeep <= o1; o += kDeep) {
+            float x[kDeep];
+#pragma unroll
+            for (int k = 0; k < kDeep; ++k) x[k] = part[(int64_t)(o + k) * count];
+#pragma unroll
+            for (int k = 0; k < kDeep; ++k) acc += x[k];
+        }
+        for (; o < o1; ++o) acc += part[(int64_t)o * count];
+        float* dst = C + (int64_t)row * N + (e - m * N);
+        *dst = accumulate ? *dst + acc : acc;
     }
 }
 
 // --------------------------------------------------------------- convert
 // fp32 [rows, cols] -> 16-bit [rows, ldo], RNE, columns cols..ldo-1 zeroed.
-// One thread writes 8 consecutive outputs (one 16-byte store); VEC reads them
-// as two 16-byte loads (cols % 8 == 0, 16-byte aligned input).
-template <bool BF16, bool VEC>
+// One thread writes 8 consecutive outputs (one 16-byte store) from two 16-byte
+// loads, which need 4-byte alignment only; scalar loads are left to the run that
+// crosses the row's end.  FLAT (ldo == cols): runs are consecutive in both.
+// Bound by its bytes: 150,000 x 100 took 31 us with scalar loads and a 64-bit
+// division per run, 18.5 us so (91 MB); 512,000 x 256 119 us either way
+// (786 MB, 6.6 TB/s).
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <bool BF16>
+__device__ __forceinline__ u16x8 convert8(const float (&x)[8]) {
+    u16x8 o;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        if constexpr (BF16) o[i] = __builtin_bit_cast(unsigned short, static_cast<__bf16>(x[i]));
+        else o[i] = __builtin_bit_cast(unsigned short, static_cast<_Float16>(x[i]));
+    }
+    return o;
+}
+
+template <bool BF16, bool FLAT, typename Index>
 __global__ __launch_bounds__(kBlock) void convert_kernel(const float* __restrict__ in,
-                                                         uint16_t* __restrict__ out, int64_t rows,
-                                                         int cols, int ldo) {
-    const int groups = ldo / 8;
-    const int64_t total = rows * groups;
-    for (int64_t g = (int64_t)blockIdx.x * kBlock + threadIdx.x; g < total;
-         g += (int64_t)gridDim.x * kBlock) {
-        const int64_t r = g / groups;
-        const int c0 = static_cast<int>(g - r * groups) * 8;
-        const float* src = in + r * cols;
+                                                         uint16_t* __restrict__ out, Index total,
+                                                         int cols, int groups) {
+    for (Index g = (Index)blockIdx.x * kBlock + threadIdx.x; g < total; g += (Index)gridDim.x * kBlock) {
+        const float* src = in + (int64_t)g * 8;
+        int left = 8;
+        if constexpr (!FLAT) {
+            const Index r = g / static_cast<Index>(groups);
+            const int c0 = static_cast<int>(g - r * static_cast<Index>(groups)) * 8;
+            src = in + (int64_t)r * cols + c0;
+            left = cols - c0;
+        }
         float x[8];
-        if constexpr (VEC) {
-            const f32x4 lo = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + c0));
-            const f32x4 hi = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + c0 + 4));
+        if (left >= 8) {
+            const f32x4u lo = __builtin_nontemporal_load(reinterpret_cast<const f32x4u*>(src));
+            const f32x4u hi = __builtin_nontemporal_load(reinterpret_cast<const f32x4u*>(src + 4));
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 x[i] = lo[i];
@@ -625,29 +656,27 @@ __global__ __launch_bounds__(kBlock) void convert_kernel(const float* __restrict
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) x[i] = (c0 + i < cols) ? src[c0 + i] : 0.f;
+            for (int i = 0; i < 8; ++i) x[i] = i < left ? src[i] : 0.f;
         }
-        u16x8 o;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            if constexpr (BF16) o[i] = __builtin_bit_cast(unsigned short, static_cast<__bf16>(x[i]));
-            else o[i] = __builtin_bit_cast(unsigned short, static_cast<_Float16>(x[i]));
-        }
-        *reinterpret_cast<u16x8*>(out + r * ldo + c0) = o;
+        *reinterpret_cast<u16x8*>(out + (int64_t)g * 8) = convert8<BF16>(x);
     }
 }
 
 ra_status launch_convert(const float* in, void* out, int64_t rows, int32_t cols, int32_t ldo,
                          bool bf16, hipStream_t st) {
     if (rows <= 0 || ldo <= 0) return RA_OK;
-    const int64_t total = rows * (ldo / 8);
+    const int groups = ldo / 8;
+    const int64_t total = rows * groups;
     const int blocks = static_cast<int>(std::min<int64_t>((total + kBlock - 1) / kBlock, 1 << 16));
-    const bool vec = (cols % 8 == 0) && ldo == cols && ra::aligned16(in);
     uint16_t* o = static_cast<uint16_t*>(out);
-    if (bf16 && vec) convert_kernel<true, true><<<blocks, kBlock, 0, st>>>(in, o, rows, cols, ldo);
-    else if (bf16) convert_kernel<true, false><<<blocks, kBlock, 0, st>>>(in, o, rows, cols, ldo);
-    else if (vec) convert_kernel<false, true><<<blocks, kBlock, 0, st>>>(in, o, rows, cols, ldo);
-    else convert_kernel<false, false><<<blocks, kBlock, 0, st>>>(in, o, rows, cols, ldo);
+    auto run = [&](auto kernel, auto n) { kernel<<<blocks, kBlock, 0, st>>>(in, o, n, cols, groups); };
+    // 32-bit run numbers, with room for the last step of the grid.
+    const bool small = total < (int64_t{1} << 31);
+    const uint32_t n32 = static_cast<uint32_t>(total);
+    if (ldo == cols && small) run(bf16 ? convert_kernel<true, true, uint32_t> : convert_kernel<false, true, uint32_t>, n32);
+    else if (ldo == cols) run(bf16 ? convert_kernel<true, true, int64_t> : convert_kernel<false, true, int64_t>, total);
+    else if (small) run(bf16 ? convert_kernel<true, false, uint32_t> : convert_kernel<false, false, uint32_t>, n32);
+    else run(bf16 ? convert_kernel<true, false, int64_t> : convert_kernel<false, false, int64_t>, total);
     RA_LAUNCH_CHECK("convert_kernel");
     return RA_OK;
 }
