@@ -748,7 +748,7 @@ Items plan_items(const ra_tile_plan* p, const Part& part) {
 // How one launch runs: columns per lane, the grid and the scheduling order.
 struct TileLaunch {
     Items items;
-    int cpl, nslices, order, lds;
+    int cpl, nslices, order;
     dim3 grid;
     int vec_store;
     float unscale;
@@ -759,7 +759,7 @@ double gathered_bytes(const ra_tile_plan* p, int N) {
     const int vb = p->info.rows_per_window == ra::kTileWindow ? ra::kTileVec : 32;
     return 2.0 * N * vb * p->info.num_blocks / std::max(p->info.col_parts, 1);
 }
-constexpr double kGatherBound = 2.0 * (1u << 30);
+constexpr double kGatherBound = 1.75 * (1u << 30);
 
 // Items of one launch that a whole workgroup shares.
 // All of them where the launch leaves much of the chip idle (fewer than 4096
@@ -772,7 +772,7 @@ constexpr double kGatherBound = 2.0 * (1u << 30);
 // Otherwise the long ones, whose chains of gathers (128 steps of ~0.6 us in a
 // window of 512 blocks) outlast the rest of a small launch: 50,000 rows of 80 at
 // N = 128 91 -> 84 us, 20,000 of 60 at N = 64 42 -> 21.  Where the gathered bytes
-// take longer than any chain (2 GiB, ~250 us) it only spreads the columns that
+// take longer than any chain (1.75 GiB, ~200 us) it only spreads the columns that
 // are gathered at a time: 100,000 rows of 60 at N = 256 33 -> 31 % L2 hits, 371
 // -> 387 us.
 int shared_items(const ra_tile_plan* p, const Part& part, int N, int nslices) {
@@ -781,19 +781,6 @@ int shared_items(const ra_tile_plan* p, const Part& part, int N, int nslices) {
     const double steps = static_cast<double>(p->info.num_blocks) / std::max(p->num_items, 1) / (tall ? 1 : 4);
     if (waves < (tall ? 1024 : 4096) && steps >= (tall ? 4 : 7)) return part.num_items;
     return gathered_bytes(p, N) < kGatherBound ? part.num_long : 0;
-}
-
-// LDS that holds a launch to 3 workgroups per CU.  Windows in flight together
-// sweep the columns from left to right side by side; in a gather-bound launch
-// without column partitions fewer of them keep closer together: 100,000 rows of
-// 60 at N = 256 32.5 -> 33.8 % L2 hits, 372 -> 360 us, 50,000 of 80 at N = 512 355
-// -> 341, 500,000 of 16 at N = 256 769 -> 760.  Partitioned plans (8,890 -> 8,940 us
-// on 250,000 rows of 500 at N = 512) and shorter launches (44.8 -> 49.8) lose.
-constexpr int kFewerWaves = 53000 - 16384;
-int tile_lds(const ra_tile_plan* p, int N) {
-    return p->info.rows_per_window == ra::kTileWindow && p->info.col_parts <= 1 &&
-                   gathered_bytes(p, N) >= kGatherBound
-               ? kFewerWaves : 0;
 }
 
 TileLaunch tile_launch(const ra_tile_plan* p, const Part& part, const float* C, const float* scratch, int N,
@@ -810,7 +797,6 @@ TileLaunch tile_launch(const ra_tile_plan* p, const Part& part, const float* C, 
     const int64_t groups =
         l.items.num_long + ((int64_t)part.num_items - l.items.num_long + kWavesPerBlock - 1) / kWavesPerBlock;
     l.grid = dim3(static_cast<unsigned>(groups * l.nslices));
-    l.lds = tile_lds(p, N);
     l.vec_store = (N % 4 == 0) && ra::aligned16(C) && (!scratch || ra::aligned16(scratch));
     l.unscale = std::ldexp(1.0f, -p->info.value_scale_log2);
     return l;
@@ -829,7 +815,7 @@ void launch_tile(const ra_tile_plan* p, const Part& part, const TileLaunch& l, c
     const int h = p->info.rows_per_window;
     if (h == 32) tile_mfma_tall_kernel<CPL, BF16, 2, BRows<CPL>><<<l.grid, kBlock, 0, st>>>(RA_TILE_ARGS);
     else if (h == 16) tile_mfma_tall_kernel<CPL, BF16, 1, BRows<CPL>><<<l.grid, kBlock, 0, st>>>(RA_TILE_ARGS);
-    else tile_mfma_kernel<CPL, BF16, BRows<CPL>><<<l.grid, kBlock, l.lds, st>>>(RA_TILE_ARGS);
+    else tile_mfma_kernel<CPL, BF16, BRows<CPL>><<<l.grid, kBlock, 0, st>>>(RA_TILE_ARGS);
 }
 
 template <bool BF16, template <int> class BRows>
@@ -861,12 +847,18 @@ ra_status launch_part(const ra_tile_plan* p, const Part& part, const uint16_t* B
     if (part.num_items == 0) return RA_OK;
     const bool wide = p->info.rows_per_window == 32 && tile_use_mfma32(N);
     const TileLaunch l = tile_launch(p, part, C, scratch, N, wide);
-    // Wide rows of a partitioned plan gather no faster without the branches, and
-    // the branches keep the windows in step: 250,000 rows of 500 at N = 512 8,880 us
-    // through the buffer, 8,840 through pointers (N = 128, one slice: 690 and 745 on
-    // 150,000 rows of 200).
+    // Launches of 8-row windows bound by their gathers keep the branches: windows
+    // in flight together sweep the columns side by side, and the faster their
+    // gathers leave the further they drift apart.  Buffer against pointers:
+    // 100,000 rows of 60 at N = 256 32.5 and 34.8 % L2 hits, 357 and 352 us;
+    // 250,000 of 500 at N = 512 8,880 and 8,800; 150,000 of 100 at N = 256 880 and
+    // 871.  With fewer bytes (50,000 of 80 at N = 128: 91 and 104) or a slice of B that
+    // the 4 MB of an L2 nearly hold (25,000 of 200 at N = 256: 128 and 140) it is the
+    // other way round.
+    const int64_t slice_bytes = static_cast<int64_t>(p->info.K) * std::min(N, 16 * l.cpl) * 2;
     const bool buf = half_buffer_fits(p->info.K, ldb) &&
-                     !(p->info.col_parts > 1 && l.nslices > 1 && p->info.rows_per_window == ra::kTileWindow);
+                     !(p->info.rows_per_window == ra::kTileWindow && gathered_bytes(p, N) >= kGatherBound &&
+                       slice_bytes > (int64_t{8} << 20));
     if (!wide) (buf ? launch_cpl<BF16, HalfBuffer> : launch_cpl<BF16, HalfPointer>)(p, part, l, Bh, ldb, C, scratch, N, st);
     else if (buf) tile_mfma_tall32_kernel<BF16, HalfBuffer<8>><<<l.grid, kBlock, 0, st>>>(RA_TILE_ARGS);
     else tile_mfma_tall32_kernel<BF16, HalfPointer<8>><<<l.grid, kBlock, 0, st>>>(RA_TILE_ARGS);
