@@ -112,3 +112,40 @@ def test_device_build_matches_host_random(seed):
     value_dtype = "bf16" if rng.random() < 0.3 else "fp16"
     print(f"[tile-build] random seed={seed} M={M} K={K} nnz={g.nnz} kind={kind} {value_dtype}", flush=True)
     _compare(g, kind, value_dtype, N=int(rng.choice([16, 64, 200])))
+
+
+def _window_graph(per_window, K, seed, shuffle):
+    """Windows of 32 rows with exactly per_window nonzeros, spread unevenly, duplicates and (shuffle) unsorted columns."""
+    rng = np.random.default_rng(seed)
+    deg = np.concatenate([rng.multinomial(n, rng.dirichlet(np.full(32, 0.3))) for n in per_window])[:-3]
+    rp = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    ci = rng.integers(0, K, rp[-1]).astype(np.int32)
+    if not shuffle:
+        for r in range(deg.size):
+            ci[rp[r]:rp[r + 1]].sort()
+    return S.Graph(rp, ci, rng.standard_normal(rp[-1]).astype(np.float32), deg.size, K, "windows")
+
+
+# Either side of each size that the window sort has a kernel for, and one past the largest (the global sort).
+@pytest.mark.parametrize("longest", [1, 255, 1024, 1025, 2048, 2049, 4096, 4097])
+@pytest.mark.parametrize("K", [64, 1 << 16])
+@pytest.mark.parametrize("kind", [0, 2])
+def test_window_sort_matches_host(longest, K, kind):
+    g = _window_graph([longest, longest // 2, 0, longest, longest // 3 + 4], K, seed=longest, shuffle=longest % 2 == 1)
+    _compare(g, kind, "fp16")
+
+
+# The counts behind the choice of the window height come from the same sort.
+@pytest.mark.parametrize("longest", [900, 3000, 6000])
+def test_window_height_choice(longest):
+    dense = _window_graph([longest] * 8, 96, seed=3, shuffle=False)    # rows share their columns: tall windows
+    sparse = _window_graph([longest] * 8, 1 << 18, seed=4, shuffle=False)
+    for g, tall in ((dense, True), (sparse, False)):
+        rp, ci, vl = g.torch("cuda")
+        plans = [mk(rp, ci, vl, g.M, g.K, 64) for mk in (ra_spmm.make_tc_direct_plan, ra_spmm.make_segment_hybrid_plan)]
+        assert all((p.rows_per_window > 8) == tall for p in plans), [p.rows_per_window for p in plans]
+        B = torch.randn(g.K, 64, device="cuda")
+        ref = ra_spmm.spmm_csr_baseline(rp, ci, vl, B)
+        scale = ra_spmm.spmm_csr_baseline(rp, ci, vl.abs(), B.abs())
+        for p in plans:
+            assert bool(((ra_spmm.run_tile_plan_route(p, B, "fp16") - ref).abs() <= 2.0 ** -10 * scale + 1e-30).all())
