@@ -11,6 +11,9 @@
 //   4. scans: vector ids, vectors and blocks per window, block offsets
 //   5. scatter: atox (first entry of each vector), values (first entry of each
 //      (col, slot) sums its duplicates in CSR order, scales, rounds)
+// Where every 32 rows fit a workgroup's LDS (window_sort), steps 2 to 5 are two
+// kernels instead: one sorts each window and counts its vectors, one writes its
+// blocks (window_emit).
 //   6. segment tables of the split schedule (64 blocks for SEGMENT_HYBRID,
 //      kTileDirectSplitBlocks otherwise)
 // Reference algorithm: tc/ra_tc_direct.cu:654-706, tc/ra_community_tc.cu:335-403,
@@ -62,6 +65,8 @@ __global__ void validate_csr(const int32_t* __restrict__ rowptr, const int32_t* 
 // out[1]: nonzeros of the longest window of 32 rows (0 for decreasing rows,
 // which validate_csr reports).
 constexpr int kReduceBlocks = 1024;
+constexpr int kWindowSortMax = 4096;  // nonzeros of 32 rows that one workgroup sorts
+constexpr int kCountSlots = 64;       // counters that the window sort spreads its counts over
 __global__ void abs_max_bits(const float* __restrict__ vals, const int32_t* __restrict__ rowptr, int M, int64_t base,
                              int64_t n, unsigned* __restrict__ out) {
     __shared__ unsigned part[2][kThreads / 64];
@@ -329,7 +334,7 @@ __global__ void order_items(const int32_t* __restrict__ flag, const int32_t* __r
 }
 
 __global__ void pack_totals(const int32_t* a, const int32_t* b, const int32_t* c, const int32_t* d, const int32_t* e,
-                            const int32_t* red, int32_t* out) {
+                            const int32_t* red, const unsigned long long* counts, int32_t* out) {
     if (threadIdx.x == 0) {
         out[0] = *a;
         out[1] = *b;
@@ -337,7 +342,9 @@ __global__ void pack_totals(const int32_t* a, const int32_t* b, const int32_t* c
         out[3] = *d;
         out[4] = *e;
         out[5] = red[0];
-        out[6] = red[1];
+        unsigned long long stored = 0;
+        for (int i = 0; counts && i < kCountSlots; ++i) stored += counts[i * 3 + 1];
+        out[6] = counts ? static_cast<int32_t>(stored) : red[1];
     }
 }
 
@@ -367,15 +374,13 @@ ra_status read_back(T* dst, const T* src, size_t n, hipStream_t st) {
 // global sort is, so the keys and values come out identical.
 // COUNT: every `every`-th 32-row window only, counting its distinct (row / h,
 // column) pairs for h = 8, 16, 32 into one of kCountSlots triples.
-constexpr int kWindowSortMax = 4096;
-constexpr int kCountSlots = 64;
 
 template <int ITEMS, bool COUNT>
 __global__ __launch_bounds__(kThreads) void window_sort(const int32_t* __restrict__ rowptr,
                                                         const int32_t* __restrict__ colind,
                                                         const float* __restrict__ vals, int M, int64_t base, int sb,
-                                                        int cb, int every, uint64_t* __restrict__ keys_out,
-                                                        float* __restrict__ vals_out,
+                                                        int cb, int every, uint32_t* __restrict__ keys_out,
+                                                        float* __restrict__ vals_out, int32_t* __restrict__ nvec,
                                                         unsigned long long* __restrict__ counts) {
     typedef hipcub::BlockRadixSort<uint32_t, kThreads, ITEMS, float> PairSort;
     typedef hipcub::BlockRadixSort<uint32_t, kThreads, ITEMS> KeySort;
@@ -393,7 +398,10 @@ __global__ __launch_bounds__(kThreads) void window_sort(const int32_t* __restric
     if (threadIdx.x <= rows) start[threadIdx.x] = rowptr[min(first + threadIdx.x, (int64_t)M)] - p0;
     __syncthreads();
     const int count = start[rows];
-    if (count == 0) return;
+    if (count == 0) {
+        if (!COUNT && threadIdx.x == 0) nvec[w] = 0;
+        return;
+    }
     uint32_t key[ITEMS];
     float val[ITEMS];
     int slot = 0;
@@ -408,58 +416,155 @@ __global__ __launch_bounds__(kThreads) void window_sort(const int32_t* __restric
             if (!COUNT) val[i] = vals[(int64_t)p0 + t];
         }
     }
-    if constexpr (!COUNT) {
-        PairSort(tmp.pairs).SortBlockedToStriped(key, val, 0, cb + sb);
-        const int64_t out = (int64_t)p0 - base;
+    if constexpr (COUNT) KeySort(tmp.keys).SortBlockedToStriped(key, 0, cb + sb);
+    else PairSort(tmp.pairs).SortBlockedToStriped(key, val, 0, cb + sb);
+    __syncthreads();
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            const int t = i * kThreads + threadIdx.x;
-            if (t < count) {
-                keys_out[out + t] = (static_cast<uint64_t>(w) << (cb + sb)) | key[i];
-                vals_out[out + t] = val[i];
-            }
-        }
-    } else {
-        KeySort(tmp.keys).SortBlockedToStriped(key, 0, cb + sb);
-        __syncthreads();
+    for (int i = 0; i < ITEMS; ++i) tmp.sorted[i * kThreads + threadIdx.x] = key[i];
+    __syncthreads();
+    // COUNT: distinct (row / h, column) pairs for h = 8, 16, 32.  Otherwise the
+    // window's vectors (c[0]) and stored entries (c[1]).
+    unsigned long long c[3] = {0, 0, 0};
+    const int64_t out = (int64_t)p0 - base;
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) tmp.sorted[i * kThreads + threadIdx.x] = key[i];
-        __syncthreads();
-        unsigned long long c[3] = {0, 0, 0};
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            const int t = i * kThreads + threadIdx.x;
-            if (t >= count) continue;
-            const uint32_t prev = t ? tmp.sorted[t - 1] : 0u;
-            const bool fresh = t == 0 || (prev >> 5) != (key[i] >> 5);
+    for (int i = 0; i < ITEMS; ++i) {
+        const int t = i * kThreads + threadIdx.x;
+        if (t >= count) continue;
+        const uint32_t prev = t ? tmp.sorted[t - 1] : 0u;
+        const bool fresh = t == 0 || (prev >> sb) != (key[i] >> sb);
+        if constexpr (COUNT) {
             c[0] += fresh || ((prev & 31) >> 3) != ((key[i] & 31) >> 3);
             c[1] += fresh || ((prev & 31) >> 4) != ((key[i] & 31) >> 4);
             c[2] += fresh;
+        } else {
+            keys_out[out + t] = key[i];
+            vals_out[out + t] = val[i];
+            c[0] += fresh;
+            c[1] += t == 0 || prev != key[i];
         }
-        for (int h = 0; h < 3; ++h) {
-            unsigned long long v = c[h];
-            for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-            if ((threadIdx.x & 63) == 0) sum[h][threadIdx.x >> 6] = v;
-        }
+    }
+    for (int h = 0; h < 3; ++h) {
+        unsigned long long v = c[h];
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        if ((threadIdx.x & 63) == 0) sum[h][threadIdx.x >> 6] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        unsigned long long v = 0;
+        for (int i = 0; i < kThreads / 64; ++i) v += sum[threadIdx.x][i];
+        if (!COUNT && threadIdx.x == 0) nvec[w] = static_cast<int32_t>(v);
+        else atomicAdd(&counts[(blockIdx.x % kCountSlots) * 3 + threadIdx.x], v);
+    }
+}
+
+// The blocks of one window from its sorted entries: vector numbers by a scan
+// over the workgroup, values gathered in LDS a stage of blocks at a time and
+// written, zeros included, as 16-byte runs; padding indices -1.  Scattering
+// 2-byte values over a zeroed array wrote every line twice: 1.6e7 nonzeros, 546
+// MB of blocks, 306 us and 68 us for the zeros, 214 us so.
+template <int ITEMS>
+__global__ __launch_bounds__(kThreads) void window_emit(const int32_t* __restrict__ rowptr, int M, int64_t base,
+                                                        const uint32_t* __restrict__ keys,
+                                                        const float* __restrict__ svals,
+                                                        const int32_t* __restrict__ block_offsets, float vscale,
+                                                        int bf16, Layout L, int32_t* __restrict__ atox,
+                                                        uint16_t* __restrict__ vals) {
+    constexpr int kStage = 8192;  // values a stage: whole blocks (64 or 32 * rows values)
+    __shared__ uint32_t s_key[ITEMS * kThreads];
+    __shared__ float s_val[ITEMS * kThreads];
+    __shared__ alignas(16) uint16_t stage[kStage];
+    __shared__ int wave_sum[kThreads / 64];
+    const int64_t w = blockIdx.x;
+    const int rows = 1 << L.sb;
+    const int64_t first = w << L.sb;
+    const int32_t p0 = rowptr[first];
+    const int count = rowptr[min(first + rows, (int64_t)M)] - p0;
+    const int b0 = block_offsets[w], nb = block_offsets[w + 1] - b0;
+    if (nb == 0) return;
+    const int64_t in = (int64_t)p0 - base;
+    for (int t = threadIdx.x; t < count; t += kThreads) {
+        s_key[t] = keys[in + t];
+        s_val[t] = svals[in + t];
+    }
+    __syncthreads();
+    // Entries t0..t0+ITEMS-1 of this thread, and the vectors that begin before them.
+    const int t0 = threadIdx.x * ITEMS;
+    int begins = 0;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const int t = t0 + i;
+        begins += t < count && (t == 0 || (s_key[t - 1] >> L.sb) != (s_key[t] >> L.sb));
+    }
+    int scan = begins;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(scan, off, 64);
+        if ((threadIdx.x & 63) >= off) scan += o;
+    }
+    if ((threadIdx.x & 63) == 63) wave_sum[threadIdx.x >> 6] = scan;
+    __syncthreads();
+    int before = scan - begins, total = 0;
+    for (int i = 0; i < kThreads / 64; ++i) {
+        if (i < static_cast<int>(threadIdx.x >> 6)) before += wave_sum[i];
+        total += wave_sum[i];
+    }
+    // Column indices; at[i] = place of the entry's value in the window, or -1
+    // where an earlier entry of the same (column, slot) holds the sum.
+    int at[ITEMS];
+    uint16_t half[ITEMS];
+    int vec = before - 1;
+    int32_t* x = atox + (int64_t)b0 * L.vb;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const int t = t0 + i;
+        at[i] = -1;
+        if (t >= count) continue;
+        const uint32_t k = s_key[t];
+        const bool fresh = t == 0 || (s_key[t - 1] >> L.sb) != (k >> L.sb);
+        if (fresh) x[++vec] = static_cast<int32_t>(k >> L.sb);
+        if (!fresh && s_key[t - 1] == k) continue;
+        float acc = 0.f + s_val[t];
+        for (int j = t + 1; j < count && s_key[j] == k; ++j) acc += s_val[j];  // duplicates, in CSR order
+        const int slot = static_cast<int>(k & static_cast<uint32_t>(rows - 1)), kk = vec % L.vb, blk = vec / L.vb;
+        at[i] = L.vb == 8 ? blk * 64 + slot * 8 + kk
+                          : blk * rows * 32 + (((slot >> 4) * 4 + (kk >> 3)) * 16 + (slot & 15)) * 8 + (kk & 7);
+        half[i] = bf16 ? ra::bf16_rne_bits(acc) : ra::half_rne_bits(acc * vscale);
+    }
+    for (int v = total + threadIdx.x; v < nb * L.vb; v += kThreads) x[v] = -1;
+    const int size = nb * rows * L.vb;  // values of the window
+    uint16_t* dst = vals + (int64_t)b0 * rows * L.vb;
+    for (int s0 = 0; s0 < size; s0 += kStage) {
+        const int len = min(kStage, size - s0);
+        for (int i = threadIdx.x; i < len / 8; i += kThreads)
+            reinterpret_cast<uint4*>(stage)[i] = make_uint4(0, 0, 0, 0);
         __syncthreads();
-        if (threadIdx.x < 3) {
-            unsigned long long v = 0;
-            for (int i = 0; i < kThreads / 64; ++i) v += sum[threadIdx.x][i];
-            atomicAdd(&counts[(blockIdx.x % kCountSlots) * 3 + threadIdx.x], v);
-        }
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i)
+            if (at[i] >= s0 && at[i] < s0 + len) stage[at[i] - s0] = half[i];
+        __syncthreads();
+        for (int i = threadIdx.x; i < len / 8; i += kThreads)
+            reinterpret_cast<uint4*>(dst + s0)[i] = reinterpret_cast<const uint4*>(stage)[i];
+        __syncthreads();
     }
 }
 
 // Items per thread for windows of up to `longest` nonzeros.
 template <bool COUNT>
 void launch_window_sort(int longest, int64_t windows, hipStream_t st, const int32_t* rowptr, const int32_t* colind,
-                        const float* vals, int M, int64_t base, int sb, int cb, int every, uint64_t* keys, float* fvals,
-                        unsigned long long* counts) {
+                        const float* vals, int M, int64_t base, int sb, int cb, int every, uint32_t* keys, float* fvals,
+                        int32_t* nvec, unsigned long long* counts) {
     auto f = longest <= 4 * kThreads    ? window_sort<4, COUNT>
              : longest <= 8 * kThreads  ? window_sort<8, COUNT>
                                         : window_sort<16, COUNT>;
     f<<<static_cast<unsigned>((windows + every - 1) / every), kThreads, 0, st>>>(rowptr, colind, vals, M, base, sb, cb,
-                                                                                 every, keys, fvals, counts);
+                                                                                 every, keys, fvals, nvec, counts);
+}
+
+void launch_window_emit(int longest, int64_t windows, hipStream_t st, const int32_t* rowptr, int M, int64_t base,
+                        const uint32_t* keys, const float* svals, const int32_t* boff, float vscale, bool bf16, Layout L,
+                        int32_t* atox, uint16_t* vals) {
+    auto f = longest <= 4 * kThreads ? window_emit<4> : longest <= 8 * kThreads ? window_emit<8> : window_emit<16>;
+    f<<<static_cast<unsigned>(windows), kThreads, 0, st>>>(rowptr, M, base, keys, svals, boff, vscale, bf16 ? 1 : 0, L,
+                                                           atox, vals);
 }
 
 // Window height for rows_per_window = 0, from the distinct (row / h, column)
@@ -555,6 +660,7 @@ ra_status gpu_build(ra_tile_plan* p, int32_t kind, const int32_t* rowptr, const 
     void* tmp = s.take<char>(tmp_bytes, off);
     uint64_t* keys = s.take<uint64_t>(nn, off);
     uint64_t* keys2 = s.take<uint64_t>(nn, off);
+    uint32_t* wkeys = reinterpret_cast<uint32_t*>(keys2);  // the window sort's keys
     float* fval = s.take<float>(nn, off);   // values in CSR order, then sorted with the keys
     float* fval2 = s.take<float>(nn, off);
     int32_t* newvec = s.take<int32_t>(nn, off);
@@ -642,7 +748,7 @@ ra_status gpu_build(ra_tile_plan* p, int32_t kind, const int32_t* rowptr, const 
             fill_u32<<<1, kThreads, 0, st>>>(reinterpret_cast<unsigned*>(layout_counts), 6 * kCountSlots);
             if (sort_windows) {
                 launch_window_sort<true>(longest, W32, st, rowptr, colind, vals, M, base, 5, cb, S, nullptr, nullptr,
-                                         layout_counts);
+                                         nullptr, layout_counts);
             } else if (S == 1) {
                 entry_keys<<<grid_for(n), kThreads, 0, st>>>(row_of, colind, vals, pos_ptr, base, n, 5, cb, INT32_MAX,
                                                              W32, keys, nullptr);
@@ -698,7 +804,9 @@ ra_status gpu_build(ra_tile_plan* p, int32_t kind, const int32_t* rowptr, const 
     if (n > 0) {
         size_t tb = tmp_bytes;
         if (sort_windows) {
-            launch_window_sort<false>(longest, W, st, rowptr, colind, vals, M, base, L.sb, L.cb, 1, keys2, fval2, nullptr);
+            fill_u32<<<1, kThreads, 0, st>>>(reinterpret_cast<unsigned*>(layout_counts), 6 * kCountSlots);
+            launch_window_sort<false>(longest, W, st, rowptr, colind, vals, M, base, L.sb, L.cb, 1, wkeys, fval2, nvec,
+                                      layout_counts);
             RA_LAUNCH_CHECK("window_sort");
         } else {
             entry_keys<<<grid_for(n), kThreads, 0, st>>>(row_of, colind, vals, pos_ptr, base, n, L.sb, L.cb,
@@ -706,15 +814,22 @@ ra_status gpu_build(ra_tile_plan* p, int32_t kind, const int32_t* rowptr, const 
             RA_HIP_TRY(hipcub::DeviceRadixSort::SortPairs(tmp, tb, keys, keys2, fval, fval2, static_cast<int>(n),
                                                           0, wshift + wbits, st));
         }
-        mark_new<<<grid_for(n), kThreads, 0, st>>>(keys2, n, L.sb, newvec, newkey);
-        tb = tmp_bytes;
-        RA_HIP_TRY(hipcub::DeviceScan::InclusiveSum(tmp, tb, newvec, vid, static_cast<int>(n), st));
+        if (!sort_windows) {
+            mark_new<<<grid_for(n), kThreads, 0, st>>>(keys2, n, L.sb, newvec, newkey);
+            tb = tmp_bytes;
+            RA_HIP_TRY(hipcub::DeviceScan::InclusiveSum(tmp, tb, newvec, vid, static_cast<int>(n), st));
+        }
     }
-    // nvec[w] from the last vector id of each window (no atomics): wvec_start
-    // is used as the temporary for the per-window last ids and their max-scan.
-    fill_i32<<<grid_for(NC + 1), kThreads, 0, st>>>(nvec, NC + 1, 0);
-    fill_i32<<<grid_for(NC + 1), kThreads, 0, st>>>(wvec_start, NC + 1, 0);
-    if (n > 0) {
+    // nvec[w], where the window sort has not counted it, from the last vector id
+    // of each window (no atomics): wvec_start is used as the temporary for the
+    // per-window last ids and their max-scan.
+    if (n == 0 || !sort_windows) {
+        fill_i32<<<grid_for(NC + 1), kThreads, 0, st>>>(nvec, NC + 1, 0);
+        fill_i32<<<grid_for(NC + 1), kThreads, 0, st>>>(wvec_start, NC + 1, 0);
+    } else {
+        fill_i32<<<1, kThreads, 0, st>>>(nvec + NC, 1, 0);
+    }
+    if (n > 0 && !sort_windows) {
         window_last_vid<<<grid_for(n), kThreads, 0, st>>>(keys2, vid, n, wshift, wvec_start);
         size_t tb = tmp_bytes;
         RA_HIP_TRY(hipcub::DeviceScan::InclusiveScan(tmp, tb, wvec_start, nvec, hipcub::Max(), static_cast<int>(NC), st));
@@ -744,7 +859,7 @@ ra_status gpu_build(ra_tile_plan* p, int32_t kind, const int32_t* rowptr, const 
         RA_HIP_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, tb, is_split, split_idx, wn, st));
         tb = tmp_bytes;
         RA_HIP_TRY(hipcub::DeviceReduce::Max(tmp, tb, blocks, red_out, static_cast<int>(NC), st));
-        if (n > 0) {
+        if (n > 0 && !sort_windows) {
             tb = tmp_bytes;
             RA_HIP_TRY(hipcub::DeviceReduce::Sum(tmp, tb, newkey, red_out + 1, static_cast<int>(n), st));
         } else {
@@ -755,7 +870,7 @@ ra_status gpu_build(ra_tile_plan* p, int32_t kind, const int32_t* rowptr, const 
     // longest window, stored entries.
     int32_t totals[7];
     pack_totals<<<1, 64, 0, st>>>(boff + NC, wvec_start + NC, seg_start + NC, slot_start + NC, split_idx + NC, red_out,
-                                  totals_out);
+                                  n > 0 && sort_windows ? layout_counts : nullptr, totals_out);
     RA_LAUNCH_CHECK("pack_totals");
     RA_TRY(read_back(totals, totals_out, 7, st));
     const int32_t reds[2] = {totals[5], totals[6]};
@@ -766,13 +881,18 @@ ra_status gpu_build(ra_tile_plan* p, int32_t kind, const int32_t* rowptr, const 
     // atox, values.
     RA_TRY(p->atox.allocate(std::max<int64_t>(nblocks, 1) * L.vb * sizeof(int32_t)));
     RA_TRY(p->vals.allocate(std::max<int64_t>(nblocks, 1) * block_vals * sizeof(uint16_t)));
-    fill_i32<<<grid_for(nblocks * L.vb), kThreads, 0, st>>>(p->atox.get<int32_t>(), nblocks * L.vb, -1);
-    // A block holds 64 values or a multiple: whole 16-byte runs.
-    fill_zero16<<<grid_for(nblocks * block_vals / 8), kThreads, 0, st>>>(p->vals.get<uint4>(), nblocks * block_vals / 8);
-    if (n > 0)
-        scatter_entries<<<grid_for(n), kThreads, 0, st>>>(keys2, fval2, vid, newkey, n, boff,
-                                                          wvec_start, vscale, bf16 ? 1 : 0, L,
-                                                          p->atox.get<int32_t>(), p->vals.get<uint16_t>());
+    if (n > 0 && sort_windows) {
+        launch_window_emit(longest, W, st, rowptr, M, base, wkeys, fval2, boff, vscale, bf16, L, p->atox.get<int32_t>(),
+                           p->vals.get<uint16_t>());
+    } else {
+        fill_i32<<<grid_for(nblocks * L.vb), kThreads, 0, st>>>(p->atox.get<int32_t>(), nblocks * L.vb, -1);
+        // A block holds 64 values or a multiple: whole 16-byte runs.
+        fill_zero16<<<grid_for(nblocks * block_vals / 8), kThreads, 0, st>>>(p->vals.get<uint4>(), nblocks * block_vals / 8);
+        if (n > 0)
+            scatter_entries<<<grid_for(n), kThreads, 0, st>>>(keys2, fval2, vid, newkey, n, boff,
+                                                              wvec_start, vscale, bf16 ? 1 : 0, L,
+                                                              p->atox.get<int32_t>(), p->vals.get<uint16_t>());
+    }
     RA_LAUNCH_CHECK("scatter_entries");
 
     // Segment tables.
