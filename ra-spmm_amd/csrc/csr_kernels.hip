@@ -215,6 +215,24 @@ __device__ __forceinline__ void accumulate_range(const int32_t* __restrict__ col
     }
 }
 
+// A whole row: shorter rounds where no row of the wave has more nonzeros than
+// they hold.  The gathers past a row's end cost issue slots although they load
+// nothing: a uniform graph of 10,000 rows of 2 at N = 128 took 5.1 us in rounds
+// of 16, 3.6 so (in rounds of 4 3.6); rows of 4 5.0 and 3.9.
+template <int G, int V, int U, typename P, typename Rows>
+__device__ __forceinline__ void accumulate_row(const int32_t* __restrict__ colind,
+                                               const float* __restrict__ vals, const Rows& rows,
+                                               int p0, int p1, int sl, const int (&q)[V],
+                                               P (&acc)[V], bool nt) {
+    if constexpr (U > 4) {
+        if (!__any(p1 - p0 > 4)) return accumulate_range<G, V, 4, P>(colind, vals, rows, p0, p1, sl, q, acc, nt);
+    }
+    if constexpr (U > 8) {
+        if (!__any(p1 - p0 > 8)) return accumulate_range<G, V, 8, P>(colind, vals, rows, p0, p1, sl, q, acc, nt);
+    }
+    accumulate_range<G, V, U, P>(colind, vals, rows, p0, p1, sl, q, acc, nt);
+}
+
 // As accumulate_range over entries [p0, p1) of a chunk whose (key, value) pairs
 // are in LDS, (kNone, -0) from the chunk's end on: one broadcast LDS read per
 // pair instead of a coalesced global load and a lane shuffle.
@@ -286,7 +304,7 @@ __global__ __launch_bounds__(kBlock) void csr_rows_kernel(
     for (int s = 0; s < V; ++s)
         acc[s] = resume ? load_packet<P>(crow, q[s]) : pzero<P>();
     const Rows rows(B, N);
-    accumulate_range<G, V, U, P>(colind, vals, rows, rowptr[row], rowptr[row + 1], sl, q, acc, nt != 0);
+    accumulate_row<G, V, U, P>(colind, vals, rows, rowptr[row], rowptr[row + 1], sl, q, acc, nt != 0);
 #pragma unroll
     for (int s = 0; s < V; ++s)
         store_packet(crow, q0 + s * G, q[s], acc[s], nt != 0);
@@ -427,8 +445,7 @@ __global__ __launch_bounds__(kBlock) void zo_fused_kernel(
     const int64_t idx = (gw - num_chunks) * RPW + sub;
     if (idx >= num_short) return;
     const int row = short_rows[idx];
-    accumulate_range<G, V, U, P>(colind, vals, rows, rowptr[row], rowptr[row + 1], sl, q, acc,
-                                 nt != 0);
+    accumulate_row<G, V, U, P>(colind, vals, rows, rowptr[row], rowptr[row + 1], sl, q, acc, nt != 0);
 #pragma unroll
     for (int s = 0; s < V; ++s)
         store_packet(C + (int64_t)row * ld, q0 + s * G, q[s], acc[s], nt != 0);
@@ -825,7 +842,9 @@ ra_status csr_direct_launch(const int32_t* d_rowptr, const int32_t* d_colind, co
     const bool deal = cslice > 0 || tuning().xslice;
     const int rows_per_block = kWavesPerBlock * (kWave / sh.G);
     dim3 grid((M + rows_per_block - 1) / rows_per_block, (np + sh.G * sh.V - 1) / (sh.G * sh.V));
-    const bool buf = buffer_rows_fit(K, N);
+    // Rows much shorter than a round of several packets a lane: branches skip the
+    // gathers past their ends (500,000 rows of 2 at N = 300: 324 us masked, 294 so).
+    const bool buf = buffer_rows_fit(K, N) && !(sh.V > 1 && nnz < 3 * static_cast<int64_t>(M));
     if (buf && vec) sh.U = gathers_in_flight(sh, (int64_t)grid.x * grid.y * kWavesPerBlock);
     auto launch = vec ? (buf ? launch_csr_rows<pk4, BufferRows> : launch_csr_rows<pk4, PointerRows>)
                       : (buf ? launch_csr_rows<float, BufferRows> : launch_csr_rows<float, PointerRows>);

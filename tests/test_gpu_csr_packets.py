@@ -73,6 +73,28 @@ def test_depths_of_the_gather_rounds(oracle, N, rows):
     np.testing.assert_array_equal(ra_spmm.run_zero_overhead_plan(plan, rp, ci, vl, Bd).cpu().numpy(), seq)
 
 
+# A launch of 16 gathers in flight (N = 64 and 128, few rows), one of 8 (N = 48, 40,000 rows) and several packets a lane
+# with rows of under 3 nonzeros (N = 300, over 2^16 waves).  Rows of 0..4, 0..8 and 0..9 nonzeros: a wave whose rows fit
+# a shorter round takes it.
+@pytest.mark.parametrize("longest", [4, 5, 8, 9])
+@pytest.mark.parametrize("N,rows", [(64, 1000), (128, 515), (48, 40_000), (300, 66_000)])
+def test_rounds_of_short_rows(oracle, N, rows, longest):
+    print(f"[short] N={N} rows={rows} longest={longest}", flush=True)
+    rng = np.random.default_rng(rows + longest)
+    deg = rng.integers(0, 3 if N == 300 else longest + 1, rows)
+    deg[::97] = longest
+    rowptr = np.zeros(rows + 1, np.int32)
+    np.cumsum(deg, out=rowptr[1:])
+    colind = rng.integers(0, 200, rowptr[-1]).astype(np.int32)
+    vals = rng.standard_normal(rowptr[-1]).astype(np.float32)
+    B = _B(200, N, seed=N)
+    seq = oracle.spmm_seq_f32(rowptr, colind, vals, B)
+    rp, ci, vl, Bd = (torch.from_numpy(x).cuda() for x in (rowptr, colind, vals, B))
+    np.testing.assert_array_equal(ra_spmm.spmm_csr_direct(rp, ci, vl, Bd).cpu().numpy(), seq)
+    plan = ra_spmm.make_zero_overhead_plan(rp, rows, 200)
+    np.testing.assert_array_equal(ra_spmm.run_zero_overhead_plan(plan, rp, ci, vl, Bd).cpu().numpy(), seq)
+
+
 def test_infinities_stay_in_their_rows(oracle):
     """Rounds past the end of a row gather nothing: an infinity or NaN in B reaches only the rows that refer to it."""
     g = S.random_csr(300, 200, 6.0, seed=3, empty_frac=0.1)
