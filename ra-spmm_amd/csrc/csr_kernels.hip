@@ -1,8 +1,9 @@
 // csr_kernels.hip — CSR family on 64-lane wavefronts (gfx950).
 //
 //   CSR_DIRECT         a lane group of G lanes owns one row; each lane keeps V
-//                      packets (4 columns; 1 where N < 4) of the output row, so
-//                      one wave-wide dwordx4 load gathers 64/G whole B rows.
+//                      packets (4 columns, or 1: one_column_packets) of the
+//                      output row, so one wave-wide dwordx4 load gathers 64/G
+//                      whole B rows.
 //                      (col, val) of a G-wide slice of the row are loaded
 //                      coalesced, one per lane, and broadcast with ds_bpermute.
 //   baseline           regime-free reference point: one wave per row, lanes
@@ -43,15 +44,11 @@ using ra::kChunk;
 using ra::kSoleFlag;
 
 // ------------------------------------------------------------------ packets
-// A packet is the run of output columns one lane owns: 4 floats, or 1 where
-// N < 4.  A 4-float packet needs 4-byte alignment only (a dwordx4 access on
-// gfx950 does), so any N >= 4 and any float buffer takes 16-byte accesses: the
-// row's last packet starts at N - 4, is loaded whole and stores only the
-// columns no other packet owns (own_from).  With 4-byte packets a row of N = 47
-// took a whole wave: a power-law graph of 1e6 rows and 2.6e7 nonzeros ran 1.07
-// ms at N = 47, now 0.97 ms, one of 2e5 rows 57.9 us at N = 31, now 46.5 us.
-// What is left over N = 48 (0.80 ms) is the unaligned rows' extra 64-byte
-// sectors.
+// A packet is the run of output columns one lane owns: 4 floats, or 1
+// (one_column_packets says which).  A 4-float packet needs 4-byte alignment
+// only (a dwordx4 access on gfx950 does), so it serves any N >= 4 and any float
+// buffer: the row's last packet starts at N - 4, is loaded whole and stores
+// only the columns no other packet owns (own_from).
 typedef float pk4 __attribute__((ext_vector_type(4), aligned(4)));
 
 template <typename P> __device__ __forceinline__ P pzero();
@@ -118,8 +115,6 @@ __device__ __forceinline__ P load_packet(const float* row, int col) {
 // columns.  PointerRows: 64-bit addresses, for anything larger.
 constexpr uint32_t kBufferLimit = 0xFFFF0000u;
 constexpr int kBufferRow = 16000;  // kNone + a column's byte offset stays below 2^32
-
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 struct BufferRows {
     typedef uint32_t Key;
@@ -639,7 +634,8 @@ struct LaneShape {
 };
 
 // Tuning knobs, read once per process: RA_CSR_LANES forces the lane-group
-// width (4..64), RA_CSR_UNROLL the gathers in flight per lane (4, 8 or 16),
+// width (4..64), RA_CSR_UNROLL the gathers in flight per lane (4, 8 or 16;
+// where a lane owns one packet, 4 otherwise),
 // RA_XCD_REMAP=0 turns the XCD-contiguous block order of CSR_DIRECT off
 // (RA_ZO_XCD_REMAP=1 turns it on for ZERO_OVERHEAD_CSR, where it piles the hub
 // chunks onto one XCD), RA_CSR_STREAMING=0 turns the non-temporal hints off,
@@ -674,7 +670,6 @@ const CsrTuning& tuning() {
 // Lane-group shape from the number of packets per row (per column pass).
 LaneShape pick_shape(int np, int packet_elems, int slice_elems = 0) {
     const CsrTuning& t = tuning();
-    if (packet_elems == 1) return {4, 1, 4};  // N < 4
     if (slice_elems > 0) np = std::min(np, std::max(1, slice_elems / packet_elems));
     else if (t.coltile > 0) np = std::min(np, std::max(1, t.coltile / packet_elems));
     int G;
@@ -698,11 +693,70 @@ int gathers_in_flight(const LaneShape& sh, int64_t waves) {
     return std::min(sh.G, u);
 }
 
-// C is written with streaming stores where its rows are whole aligned packets
-// (1e6 rows at N = 16: 249 -> 244 us, at N = 128: 894 -> 888 us).  Ragged rows
-// share 16-byte runs with their neighbours, which the cache should merge: N =
-// 31 streamed 52.8 us, cached 46.5 us; N = 47 992 and 974 us.
+// The index and value streams are read and C is written with the streaming hint
+// where C's rows are whole aligned packets (1e6 rows at N = 16: 249 -> 244 us, at
+// N = 128: 894 -> 888 us).  Ragged rows share 16-byte runs with their
+// neighbours, which the cache should merge: N = 31 streamed 52.8 us, cached 46.5
+// us; N = 47 992 and 974 us.
 inline bool whole_packets(const float* C, int N) { return N % 4 == 0 && ra::aligned16(C); }
+
+// What the choice of packets and slices looks at: a matrix of M rows, K columns
+// and nnz nonzeros times N columns; binned: ZERO_OVERHEAD_CSR, whose rows differ
+// much in length.
+struct RowLoad {
+    int64_t M, K, nnz;
+    int N;
+    bool ragged, binned;  // ragged: rows of B or C that are not whole aligned 16-byte runs
+};
+
+// One column a lane instead of four, on ragged rows.  Four a lane take a quarter
+// of the waves, lane permutes and instructions, but their loads straddle cache
+// sectors, so one a lane wins where the gathered bytes set the time and where
+// four would leave a group's lanes unused.  us, four / one:
+//   N <= 8: always.  300,000 rows of 20 at N = 5 63 / 51; hubs, 20,000 rows of 12
+//   16 / 10.
+//   N <= 16: unless rows are short, where waves count: 100,000 rows of 3 at N = 13
+//   8.5 / 10.8, 50,000 of 6 5.1 / 5.8, 300,000 of 20 107 / 86; hubs, 1e6 rows of 12
+//   257 / 238.
+//   N <= 32 with hub rows, whose chains get 16 gathers in flight instead of 8, or
+//   long rows: hubs, 20,000 rows of 24 at N = 30 24 / 17, 200,000 of 6 38 / 43.
+//   N <= 128 where a one-column wave gathers 3,000 bytes (2,000 from a large B of
+//   narrow rows) and B is well past the L2s: 300,000 rows of 32 at N = 30 378 / 342, of
+//   8 at N = 33 94 / 110; 30,000 of 20 at N = 33 13 / 18; 50,000 uneven rows of 15 at
+//   N = 65 55 / 69.
+//   Wider, both take the same time (100,000 rows of 20 at N = 225 229 / 229) or
+//   four win (20,000 rows of 12 with hubs 28 / 38).
+inline bool one_column_packets(const RowLoad& r) {
+    if (r.N < 4) return true;
+    if (!r.ragged || r.N > 128) return false;
+    if (r.N <= 8) return true;
+    if (r.N <= 16) return r.binned || r.nnz >= 8 * r.M;
+    if (r.binned) return r.N <= 32 && (r.M < 100000 || r.nnz >= 16 * r.M);
+    const int64_t row = r.N * int64_t{4}, B = r.K * row;
+    const int64_t wave = r.nnz * row * (r.N <= 32 ? 2 : 1);  // bytes a wave gathers, times M
+    if (r.N <= 32 && B >= 24000000) return wave >= 2000 * r.M;
+    return wave >= 3000 * r.M && B >= (r.N <= 64 ? 8000000 : 32000000);
+}
+
+// Column slice of 128 dealt to the XCDs for wide rows of four-column packets (each
+// XCD's L2 then holds half or less of every gathered B row, and a small launch
+// has 2-4x as many waves, each with a shorter chain).
+// Whole rows: from N = 256, on CSR_DIRECT below 2^16 unsliced waves (larger
+// ones only re-read A per slice: 512,000 rows at N = 512 1.91 -> 2.18 ms).
+// Ragged rows: a slice's edges cut packets and the last slice is partly empty, so
+// only small launches take slices, from 3 whole ones on (us, unsliced / sliced:
+// 10,000 rows of 20 at N = 401 40 / 31, at N = 301 29 / 35; 30,000 of 8 at N = 449 70 /
+// 75; hubs, 120,000 of 13 at N = 510 449 / 423, at N = 301 and 60,000 of 24 200 / 244,
+// 200,000 of 12 at N = 401 508 / 590), with hub rows also narrower ones of few nonzeros, bound by
+// the longest chain (20,000 of 6 at N = 301 39 / 28, of 24 62 / 71).
+inline int column_slice(const RowLoad& r, int64_t unsliced_waves) {
+    if (r.ragged) {
+        if (r.N <= 256) return 0;
+        if (r.binned) return (r.M < 25000 && (r.N > 384 || r.nnz < 16 * r.M)) || (r.M < 150000 && r.N > 440) ? 128 : 0;
+        return r.M < 16000 && r.N > 384 && r.nnz >= 4 * r.M ? 128 : 0;
+    }
+    return r.N >= 256 && (r.binned || unsliced_waves < (int64_t{1} << 16)) ? 128 : 0;
+}
 
 // B and its rows fit the 32-bit offsets of BufferRows.
 inline bool buffer_rows_fit(int64_t K, int N) { return N <= kBufferRow && K * N * 4 <= int64_t{kBufferLimit}; }
@@ -733,23 +787,19 @@ ra_status launch_csr_rows(const LaneShape& sh, dim3 grid, hipStream_t st, const 
         return RA_OK;                                                                       \
     }
 #define RA_ROWS_G(g, u) RA_ROWS_CASE(g, 1, u) RA_ROWS_CASE(g, 2, u) RA_ROWS_CASE(g, 4, u)
-    RA_ROWS_CASE(4, 1, 4)
-    if constexpr (PacketElems<P>::value == 4) {
-        RA_ROWS_CASE(4, 2, 4)
-        RA_ROWS_CASE(4, 4, 4)
-        RA_ROWS_G(8, 4)
-        RA_ROWS_G(16, 4)
-        RA_ROWS_G(32, 4)
-        RA_ROWS_G(64, 4)
-        if constexpr (std::is_same_v<Rows, BufferRows>) {
-            RA_ROWS_CASE(8, 1, 8)
-            RA_ROWS_CASE(16, 1, 8)
-            RA_ROWS_CASE(32, 1, 8)
-            RA_ROWS_CASE(64, 1, 8)
-            RA_ROWS_CASE(16, 1, 16)
-            RA_ROWS_CASE(32, 1, 16)
-            RA_ROWS_CASE(64, 1, 16)
-        }
+    RA_ROWS_G(4, 4)
+    RA_ROWS_G(8, 4)
+    RA_ROWS_G(16, 4)
+    RA_ROWS_G(32, 4)
+    RA_ROWS_G(64, 4)
+    if constexpr (std::is_same_v<Rows, BufferRows>) {
+        RA_ROWS_CASE(8, 1, 8)
+        RA_ROWS_CASE(16, 1, 8)
+        RA_ROWS_CASE(32, 1, 8)
+        RA_ROWS_CASE(64, 1, 8)
+        RA_ROWS_CASE(16, 1, 16)
+        RA_ROWS_CASE(32, 1, 16)
+        RA_ROWS_CASE(64, 1, 16)
     }
 #undef RA_ROWS_G
 #undef RA_ROWS_CASE
@@ -778,23 +828,19 @@ ra_status launch_zo(const LaneShape& sh, dim3 grid, hipStream_t st, const int32_
         return RA_OK;                                                                        \
     }
 #define RA_ZO_G(g, u) RA_ZO_CASE(g, 1, u) RA_ZO_CASE(g, 2, u) RA_ZO_CASE(g, 4, u)
-    RA_ZO_CASE(4, 1, 4)
-    if constexpr (PacketElems<P>::value == 4) {
-        RA_ZO_CASE(4, 2, 4)
-        RA_ZO_CASE(4, 4, 4)
-        RA_ZO_G(8, 4)
-        RA_ZO_G(16, 4)
-        RA_ZO_G(32, 4)
-        RA_ZO_G(64, 4)
-        if constexpr (std::is_same_v<Rows, BufferRows>) {
-            RA_ZO_CASE(8, 1, 8)
-            RA_ZO_CASE(16, 1, 8)
-            RA_ZO_CASE(32, 1, 8)
-            RA_ZO_CASE(64, 1, 8)
-            RA_ZO_CASE(16, 1, 16)
-            RA_ZO_CASE(32, 1, 16)
-            RA_ZO_CASE(64, 1, 16)
-        }
+    RA_ZO_G(4, 4)
+    RA_ZO_G(8, 4)
+    RA_ZO_G(16, 4)
+    RA_ZO_G(32, 4)
+    RA_ZO_G(64, 4)
+    if constexpr (std::is_same_v<Rows, BufferRows>) {
+        RA_ZO_CASE(8, 1, 8)
+        RA_ZO_CASE(16, 1, 8)
+        RA_ZO_CASE(32, 1, 8)
+        RA_ZO_CASE(64, 1, 8)
+        RA_ZO_CASE(16, 1, 16)
+        RA_ZO_CASE(32, 1, 16)
+        RA_ZO_CASE(64, 1, 16)
     }
 #undef RA_ZO_G
 #undef RA_ZO_CASE
@@ -825,18 +871,13 @@ ra_status csr_direct_launch(const int32_t* d_rowptr, const int32_t* d_colind, co
                             bool resume, hipStream_t st) {
     RA_TRY(check_spmm_args(d_rowptr, d_colind, d_vals, d_B, d_C, M, K, N, nnz));
     if (M == 0 || N == 0) return RA_OK;
-    const bool vec = N >= 4;
+    const RowLoad load{M, K, nnz, N, !whole_packets(d_C, N) || !ra::aligned16(d_B), false};
+    const bool vec = !one_column_packets(load);
     const int np = vec ? (N + 3) / 4 : N;
-    // Wide rows of a small matrix: 128-column slices dealt to the XCDs, as
-    // ZERO_OVERHEAD_CSR does, so that fewer than 2^16 waves (about 64 per CU)
-    // become 2-4x as many, each with a shorter chain of dependent gathers.
-    // On larger matrices the slices only re-read A per slice (config 3 at
-    // N=512: 1.91 -> 2.18 ms), so they stay off there.
     int cslice = tuning().csr_slice;
     if (cslice < 0) {
         const LaneShape whole = pick_shape(np, vec ? 4 : 1);
-        const int64_t waves = (static_cast<int64_t>(M) + kWave / whole.G - 1) / (kWave / whole.G);
-        cslice = (vec && N >= 256 && waves < (int64_t{1} << 16)) ? 128 : 0;
+        cslice = vec ? column_slice(load, (static_cast<int64_t>(M) + kWave / whole.G - 1) / (kWave / whole.G)) : 0;
     }
     LaneShape sh = pick_shape(np, vec ? 4 : 1, cslice);
     const bool deal = cslice > 0 || tuning().xslice;
@@ -845,7 +886,7 @@ ra_status csr_direct_launch(const int32_t* d_rowptr, const int32_t* d_colind, co
     // Rows much shorter than a round of several packets a lane: branches skip the
     // gathers past their ends (500,000 rows of 2 at N = 300: 324 us masked, 294 so).
     const bool buf = buffer_rows_fit(K, N) && !(sh.V > 1 && nnz < 3 * static_cast<int64_t>(M));
-    if (buf && vec) sh.U = gathers_in_flight(sh, (int64_t)grid.x * grid.y * kWavesPerBlock);
+    if (buf) sh.U = gathers_in_flight(sh, (int64_t)grid.x * grid.y * kWavesPerBlock);
     auto launch = vec ? (buf ? launch_csr_rows<pk4, BufferRows> : launch_csr_rows<pk4, PointerRows>)
                       : (buf ? launch_csr_rows<float, BufferRows> : launch_csr_rows<float, PointerRows>);
     return launch(sh, grid, st, d_rowptr, d_colind, d_vals, d_B, d_C, M, N, resume ? 1 : 0, deal);
@@ -863,11 +904,10 @@ static ra_status zo_run(ra_zo_plan* plan, const int32_t* d_rowptr, const int32_t
     const int32_t M = plan->info.M;
     RA_TRY(check_spmm_args(d_rowptr, d_colind, d_vals, d_B, d_C, M, plan->info.K, N, 0));
     if (M == 0 || N == 0) return RA_OK;
-    const bool vec = N >= 4;
+    const RowLoad load{M, plan->info.K, plan->nnz, N, !whole_packets(d_C, N) || !ra::aligned16(d_B), true};
+    const bool vec = !one_column_packets(load);
     const int np = vec ? (N + 3) / 4 : N;
-    // Wide rows are cut into 128-column slices dealt to the XCDs (each XCD's
-    // L2 then holds half or less of every gathered B row).
-    const int zslice = tuning().zo_slice >= 0 ? tuning().zo_slice : (vec && N >= 256 ? 128 : 0);
+    const int zslice = tuning().zo_slice >= 0 ? tuning().zo_slice : vec ? column_slice(load, 0) : 0;
     LaneShape sh = pick_shape(np, vec ? 4 : 1, zslice);
     if (plan->info.num_split_chunks > 0 && !partials) {
         RA_TRY(plan->partials.ensure((size_t)plan->info.num_split_chunks * N * sizeof(float)));
@@ -879,7 +919,7 @@ static ra_status zo_run(ra_zo_plan* plan, const int32_t* d_rowptr, const int32_t
     if (waves > 0 && stage != 2) {
         dim3 grid((waves + kWavesPerBlock - 1) / kWavesPerBlock, tiles);
         const bool buf = buffer_rows_fit(plan->info.K, N);
-        if (buf && vec) sh.U = gathers_in_flight(sh, waves * tiles);
+        if (buf) sh.U = gathers_in_flight(sh, waves * tiles);
         auto launch = vec ? (buf ? launch_zo<pk4, BufferRows> : launch_zo<pk4, PointerRows>)
                           : (buf ? launch_zo<float, BufferRows> : launch_zo<float, PointerRows>);
         RA_TRY(launch(sh, grid, st, d_rowptr, d_colind, d_vals, d_B, d_C, plan->chunk_rows, plan->chunk_starts,
@@ -1101,6 +1141,7 @@ ra_status ra_zo_plan_create(const int32_t* h_rowptr, int32_t M, int32_t K, ra_zo
         (s = up(plan->split_rows, split_rows)) == RA_OK && (s = up(plan->split_off, split_off)) == RA_OK) {
         plan->info = z;
         plan->num_short_total = static_cast<int64_t>(short_rows.size());
+        plan->nnz = M > 0 ? static_cast<int64_t>(h_rowptr[M]) - h_rowptr[0] : 0;
         *out = plan;
         return RA_OK;
     }

@@ -39,6 +39,7 @@ __device__ __forceinline__ int bin_of(int64_t d, int& chunks) {
 struct ZoTotals {
     int32_t c[kCounters];
     int32_t decreasing, longest;
+    int32_t nnz;  // of the whole matrix (in the totals only)
 };
 
 __device__ __forceinline__ int wave_sum(int v) {
@@ -105,7 +106,8 @@ __global__ __launch_bounds__(kThreads) void zo_count(const int32_t* __restrict__
 // One workgroup, a wave per counter (waves 8 and 9: decreasing rows and the
 // longest), 64 tiles a step.
 constexpr int kScanThreads = 64 * (kCounters + 2);
-__global__ __launch_bounds__(kScanThreads) void zo_scan(ZoTotals* __restrict__ tiles, int n, ZoTotals* __restrict__ out) {
+__global__ __launch_bounds__(kScanThreads) void zo_scan(const int32_t* __restrict__ rowptr, int M,
+                                                        ZoTotals* __restrict__ tiles, int n, ZoTotals* __restrict__ out) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     int carry = 0;
     for (int t0 = 0; t0 < n; t0 += 64) {
@@ -126,7 +128,10 @@ __global__ __launch_bounds__(kScanThreads) void zo_scan(ZoTotals* __restrict__ t
     if (lane != 0) return;
     if (wave < kCounters) out->c[wave] = carry;
     else if (wave == kCounters) out->decreasing = carry;
-    else out->longest = carry;
+    else {
+        out->longest = carry;
+        out->nnz = rowptr[M] - rowptr[0];
+    }
 }
 
 // Every row to its list: the tile's offset, plus the rows of the same bin before
@@ -227,7 +232,7 @@ ra_status gpu_bin(ra_zo_plan* p, const int32_t* rowptr, int32_t M, int32_t K, hi
     ZoTotals* counts = tmp.get<ZoTotals>();
     zo_count<<<tiles, kThreads, 0, st>>>(rowptr, M, rows_per_tile, counts);
     RA_LAUNCH_CHECK("zo_count");
-    zo_scan<<<1, kScanThreads, 0, st>>>(counts, tiles, counts + tiles);
+    zo_scan<<<1, kScanThreads, 0, st>>>(rowptr, M, counts, tiles, counts + tiles);
     RA_LAUNCH_CHECK("zo_scan");
     ZoTotals tot;
     RA_HIP_TRY(hipMemcpyAsync(&tot, counts + tiles, sizeof(tot), hipMemcpyDeviceToHost, st));
@@ -248,6 +253,7 @@ ra_status gpu_bin(ra_zo_plan* p, const int32_t* rowptr, int32_t M, int32_t K, hi
     z.plan_bytes = (int64_t)sizeof(int32_t) *
                    ((int64_t)z.num_small + z.num_empty + 3LL * z.num_chunks + 2LL * z.num_split_rows + 1);
     p->num_short_total = (int64_t)z.num_empty + z.num_small;
+    p->nnz = tot.nnz;
 
     RA_TRY(p->carve(p->num_short_total, z.num_chunks, z.num_split_rows));
     const int4 base{0, z.num_empty, z.num_empty + z.num_tiny, z.num_empty + z.num_tiny + z.num_short};

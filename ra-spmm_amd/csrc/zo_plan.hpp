@@ -32,6 +32,7 @@ struct ra_zo_plan {
             *split_rows = nullptr, *split_off = nullptr;
     ra::DeviceBuffer partials;  // grown per N, reused across runs
     int64_t num_short_total = 0; // empty + tiny + short + medium
+    int64_t nnz = 0;
 
     ra_status carve(int64_t n_short, int64_t n_chunks, int64_t n_split) {
         const int64_t counts[6] = {n_short, n_chunks, n_chunks, n_chunks, n_split, n_split + 1};

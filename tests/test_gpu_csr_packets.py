@@ -1,4 +1,4 @@
-"""16-byte packets at any width N and alignment, and the depth of the gather rounds.
+"""Packets of four columns and of one at any width N and alignment, and the depth of the gather rounds.
 
 A row's last packet starts at column N - 4 and stores only the columns that no
 other packet owns; launches of fewer waves keep more gathers in flight.  Neither
@@ -21,7 +21,7 @@ def _B(K, N, seed):
     return np.random.default_rng(seed).standard_normal((K, N)).astype(np.float32)
 
 
-# 1-3: scalar packets; 4-9, 15-17: one to five packets; 63-65, 127-129: lane-group edges; 253-259: column slices.
+# 1-3: one column a lane, as where ragged rows are narrow; 4-9, 15-17: one to five packets; 63-65, 127-129: lane-group edges; 253-259: column slices.
 @pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 6, 7, 9, 15, 17, 31, 33, 63, 65, 127, 129, 253, 257, 259, 510, 1001])
 @pytest.mark.parametrize("shift", [0, 1, 2])
 def test_every_width_and_alignment(oracle, N, shift):
@@ -41,6 +41,29 @@ def test_every_width_and_alignment(oracle, N, shift):
     np.testing.assert_array_equal(C[deg <= 256], seq[deg <= 256])
     assert_close_scaled(C, oracle.spmm_f64(g.rowptr, g.colind, g.vals, B),
                         oracle.spmm_f64(g.rowptr, g.colind, np.abs(g.vals), np.abs(B)), 1e-5, f"zo N={N}")
+
+
+# Ragged widths at the bounds of the rule for one column a lane (N = 8, 16, 32, 128; mean row 8, 16; 3,000 bytes a wave and
+# 8 MB of B) and of the rule for slices (N = 385, 441; 16,000 and 25,000 rows).
+@pytest.mark.parametrize("rows,mean,widths", [(2000, 3.0, (9, 13, 401)), (2000, 10.0, (8, 11, 17, 31)), (2000, 18.0, (30, 33, 127)),
+                                              (17_000, 14.0, (126, 130, 385)), (26_000, 3.0, (301, 441))])
+def test_packets_and_slices_of_ragged_rows(oracle, rows, mean, widths):
+    g = S.random_csr(rows, rows, mean, seed=rows, skew=0.9, empty_frac=0.02, max_deg=700)
+    deg = np.diff(g.rowptr)
+    rp, ci, vl = g.torch("cuda")
+    plan = ra_spmm.make_zero_overhead_plan(rp, g.M, g.K)
+    host = ra_spmm.make_zero_overhead_plan(rp.cpu(), g.M, g.K, build="host")
+    for N in widths:
+        print(f"[ragged] rows={rows} N={N}", flush=True)
+        B = _B(g.K, N, seed=N)
+        seq = oracle.spmm_seq_f32(g.rowptr, g.colind, g.vals, B)
+        Bd = torch.from_numpy(B).cuda()
+        np.testing.assert_array_equal(ra_spmm.spmm_csr_direct(rp, ci, vl, Bd).cpu().numpy(), seq)
+        C = ra_spmm.run_zero_overhead_plan(plan, rp, ci, vl, Bd).cpu().numpy()
+        np.testing.assert_array_equal(ra_spmm.run_zero_overhead_plan(host, rp, ci, vl, Bd).cpu().numpy(), C)
+        np.testing.assert_array_equal(C[deg <= 256], seq[deg <= 256])
+        assert_close_scaled(C, oracle.spmm_f64(g.rowptr, g.colind, g.vals, B),
+                            oracle.spmm_f64(g.rowptr, g.colind, np.abs(g.vals), np.abs(B)), 1e-5, f"zo N={N}")
 
 
 @pytest.mark.parametrize("N", [47, 129, 258])
