@@ -351,7 +351,9 @@ ra_status ra_tile_plan_create_device(int32_t kind, const int32_t* d_rowptr, cons
                                      const float* d_vals, int32_t M, int32_t K, int32_t N,
                                      int32_t value_dtype, int32_t rows_per_window, ra_stream_t stream,
                                      ra_tile_plan** out);
-/* Copy a plan array back to the host (same names as ra_tile_host_export). */
+/* Copy a plan array back to the host: the names of ra_tile_host_export, and
+ * "item_order", the segments in launch order where the plan has long ones (empty
+ * otherwise). */
 ra_status ra_tile_plan_export(const ra_tile_plan* plan, const char* name, void* dst,
                               int64_t* count);
 /* B fp32 [K,N]; route: ra_tile_route.  The FP16/BF16 routes convert B into

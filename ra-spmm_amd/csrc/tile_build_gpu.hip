@@ -921,10 +921,11 @@ ra_status gpu_build(ra_tile_plan* p, int32_t kind, const int32_t* rowptr, const 
     p->part_items[P] = static_cast<int32_t>(nseg);
     p->part_splits[P] = static_cast<int32_t>(nsplit);
 
-    // Launch order, where some item is long (128 blocks of 8 vectors).
+    // Launch order, where some item (a window, or a segment of `limit` blocks) is
+    // long (128 blocks of 8 vectors): never in SEGMENT_HYBRID.
     p->part_long.assign(P, 0);
     const int long_blocks = ra::kTileLongBlocks * ra::kTileVec / L.vb;
-    p->has_long = reds[0] > long_blocks;
+    p->has_long = std::min(reds[0], limit) > long_blocks;
     if (p->has_long) {
         size_t scan6 = 0;
         RA_HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, scan6, inull, inull, static_cast<int>(nseg + 1), st));
@@ -981,6 +982,7 @@ const ra::DeviceBuffer* plan_array(const ra_tile_plan* p, const std::string& n, 
     if (n == "seg_window") { count = I.num_segments; return &p->seg_window; }
     if (n == "seg_bbegin") { count = I.num_segments; return &p->seg_bbegin; }
     if (n == "seg_bend") { count = I.num_segments; return &p->seg_bend; }
+    if (n == "item_order") { count = p->has_long ? I.num_segments : 0; return &p->item_order; }
     if (n == "seg_slot") { count = I.num_segments; return &p->seg_slot; }
     if (n == "split_windows") { count = I.num_split_windows; return &p->split_windows; }
     if (n == "split_offsets") { count = I.active ? I.num_split_windows + 1 : 0; return &p->split_offsets; }

@@ -44,8 +44,9 @@ constexpr int kTileSegBlocks = 64;    // SEGMENT_HYBRID: max blocks per segment
 // thousands of blocks while the rest of the GPU idles.
 constexpr int kTileDirectSplitBlocks = 512;
 constexpr uint32_t kTileSoleFlag = 0x80000000u;
-// Items (segments) of more blocks than this are run first, each by a whole
-// workgroup.
+// Items (segments) of more blocks than this (of 8 vectors; a quarter of it in
+// blocks of 32) come first in the launch order, and a whole workgroup may run
+// each (shared_items in tile_kernels.hip).
 constexpr int kTileLongBlocks = 128;
 
 uint16_t f32_to_f16_rne(float f);

@@ -62,3 +62,20 @@ def test_long_items_first(oracle, monkeypatch, length, parts, build):
     plan = _check(oracle, g, 0, 64, 8, build=build)
     assert plan.num_segments * plan.col_parts > 2048
     _check(oracle, g, 1, 40, 8, build=build)
+
+
+def test_order_only_where_items_are_long():
+    """A window of SEGMENT_HYBRID is cut into segments that are never long: its plan has no launch order of its own,
+    however long the window.  A whole window of TC_DIRECT comes first."""
+    g = _long_rows(1700, 2500, 1500, 1600, seed=9)
+    rp, ci, vl = g.torch("cuda")
+    for rows in (8, 32):
+        plan = ra_spmm.make_segment_hybrid_plan(rp, ci, vl, g.M, g.K, 64, rows_per_window=rows)
+        assert plan.max_window_blocks * (8 if rows == 8 else 32) > 1024
+        assert ra_spmm.export_tile_plan(plan, "item_order").numel() == 0
+        plan = ra_spmm.make_tc_direct_plan(rp, ci, vl, g.M, g.K, 64, rows_per_window=rows)
+        first = sorted({0, 1500 // rows})
+        rest = [w for w in range(plan.num_windows) if w not in first]
+        assert ra_spmm.export_tile_plan(plan, "item_order").tolist() == first + rest
+    host = ra_spmm.make_segment_hybrid_plan(*(t.cpu() for t in (rp, ci, vl)), g.M, g.K, 64, build="host")
+    assert ra_spmm.export_tile_plan(host, "item_order").numel() == 0
