@@ -746,7 +746,7 @@ inline bool one_column_packets(const RowLoad& r) {
 // Ragged rows: a slice's edges cut packets and the last slice is partly empty, so
 // only small launches take slices, from 3 whole ones on (us, unsliced / sliced:
 // 10,000 rows of 20 at N = 401 40 / 31, at N = 301 29 / 35; 30,000 of 8 at N = 449 70 /
-// 75; hubs, 120,000 of 13 at N = 510 449 / 423, at N = 301 and 60,000 of 24 200 / 244,
+// 75; hubs, 120,000 of 13 at N = 510 449 / 423, 60,000 of 24 at N = 301 200 / 244,
 // 200,000 of 12 at N = 401 508 / 590), with hub rows also narrower ones of few nonzeros, bound by
 // the longest chain (20,000 of 6 at N = 301 39 / 28, of 24 62 / 71).
 inline int column_slice(const RowLoad& r, int64_t unsliced_waves) {

@@ -761,26 +761,52 @@ double gathered_bytes(const ra_tile_plan* p, int N) {
 }
 constexpr double kGatherBound = 1.75 * (1u << 30);
 
+// Blocks of the plan's longest item over those of its mean one.
+double item_skew(const ra_tile_plan* p) {
+    const int vb = p->info.rows_per_window == ra::kTileWindow ? ra::kTileVec : 32;
+    const int limit =
+        (p->info.kind == RA_TILE_SEGMENT_HYBRID ? ra::kTileSegBlocks : ra::kTileDirectSplitBlocks) * ra::kTileVec / vb;
+    return static_cast<double>(std::min(p->info.max_window_blocks, limit)) * std::max(p->num_items, 1) /
+           std::max(p->info.num_blocks, 1);
+}
+
+// Waves of the kernel that the chip holds at once (registers: 8 and 16 rows 51-56,
+// 74 and 109 at 1-2, 4 and 8 columns a lane, 32 rows 56, 72, 98 and 140).
+int64_t resident_waves(const ra_tile_plan* p, int cpl) {
+    constexpr int kCus = 256;
+    if (p->info.rows_per_window == 32) return kCus * (cpl == 1 ? 32 : cpl == 2 ? 28 : cpl == 4 ? 20 : 12);
+    return kCus * (cpl <= 2 ? 32 : cpl == 4 ? 28 : 16);
+}
+
 // Items of one launch that a whole workgroup shares.
-// All of them where the launch leaves much of the chip idle (fewer than 4096
-// waves; 1024 of tall windows, which hold more registers) and a quarter is worth
-// a wave: 15,000 rows of degree 30 at N = 64 (1.9e3 items of 7.5 steps) 17.9 -> 16.3
-// us, 30,000 of 200 at N = 128 (3.8e3 of 50) 87 -> 79, a community graph of 8,000
-// rows at N = 128 (250 tall items) 18.4 -> 9.0.  With shorter items it loses (10,000
-// rows of 22 at N = 176, 5.5 steps: 17.0 -> 19.4), and with more tall ones (64,000
-// rows: 43.6 -> 55.6).
-// Otherwise the long ones, whose chains of gathers (128 steps of ~0.6 us in a
-// window of 512 blocks) outlast the rest of a small launch: 50,000 rows of 80 at
-// N = 128 91 -> 84 us, 20,000 of 60 at N = 64 42 -> 21.  Where the gathered bytes
-// take longer than any chain (1.75 GiB, ~200 us) it only spreads the columns that
-// are gathered at a time: 100,000 rows of 60 at N = 256 33 -> 31 % L2 hits, 371
-// -> 387 us.
-int shared_items(const ra_tile_plan* p, const Part& part, int N, int nslices) {
+// All of them while the four times as many waves still find room: a wave then has
+// a quarter of the steps, but all of an item's prologue (its tables, the first
+// indices and keys) and the sum over LDS.  8-row windows of equal length gain up
+// to twice the resident waves (1,000 windows of 15 steps at N = 128 14.0 -> 9.8 us,
+// 2,000 of 15 18.5 -> 17.3) and lose beyond (2,600 of 7.5 15 -> 18, 4,000 of 25 44 ->
+// 68); 16-row ones up to 0.8 times, 32-row ones 0.6, where they are long 0.9 (N = 128: 500 of 16 steps
+// 16.2 -> 13.4, 500 of 8 8.6 -> 10.5, 750 of 28 20 -> 18; N = 64: 1,000 of 4 5.9 ->
+// 5.1).  The longer the longest item against the mean one, the later that is: its
+// chain would outlast the rest (3,000 8-row windows of 15 steps, the longest 4 times
+// the mean, 33 -> 24 us), until the shared ones alone do as well (5,000 of 15 at N =
+// 128 71 against 81 for all).  Items of fewer than 6 steps (4 tall) do not pay for it
+// (2,000 of 5 at N = 256 17 -> 20).
+// Otherwise the long ones, where they are exceptional (twice the mean), whose
+// chains of gathers (128 steps of ~0.6 us in a window of 512 blocks) outlast the
+// rest of a small launch: 50,000 rows of 80 at N = 128 91 -> 84 us, 20,000 of 60 at
+// N = 64 42 -> 21; of 6,000 windows of 200 blocks each all would be long (N = 64 84 ->
+// 102).  Where the gathered bytes take longer than any chain (1.75 GiB, ~200 us)
+// it only spreads the columns that are gathered at a time: 100,000 rows of 60 at N
+// = 256 33 -> 31 % L2 hits, 371 -> 387 us.
+int shared_items(const ra_tile_plan* p, const Part& part, int N, int nslices, int cpl) {
     const bool tall = p->info.rows_per_window != ra::kTileWindow;
     const int64_t waves = (int64_t)part.num_items * nslices;
     const double steps = static_cast<double>(p->info.num_blocks) / std::max(p->num_items, 1) / (tall ? 1 : 4);
-    if (waves < (tall ? 1024 : 4096) && steps >= (tall ? 4 : 7)) return part.num_items;
-    return gathered_bytes(p, N) < kGatherBound ? part.num_long : 0;
+    const double skew = item_skew(p), more = std::min(skew, 4.0) - 1.0;
+    const double room = tall ? (steps < 6 || p->info.rows_per_window == 16 ? 0.8 : 0.6 + 0.015 * std::max(steps - 8, 0.0)) + more
+                             : std::min(2.0 + 1.4 * more, 4.0);
+    if (kWavesPerBlock * waves <= room * resident_waves(p, cpl) && steps >= (tall ? 4 : 6)) return part.num_items;
+    return skew >= 2 && gathered_bytes(p, N) < kGatherBound ? part.num_long : 0;
 }
 
 TileLaunch tile_launch(const ra_tile_plan* p, const Part& part, const float* C, const float* scratch, int N,
@@ -792,7 +818,7 @@ TileLaunch tile_launch(const ra_tile_plan* p, const Part& part, const float* C, 
     const bool remap = p->info.kind != RA_TILE_COMMUNITY_TC && tile_remap();
     l.order = (remap ? 1 : 0) | (tile_slice_major(l.nslices, remap) ? 2 : 0);
     l.items = plan_items(p, part);
-    l.items.num_long = wide ? 0 : shared_items(p, part, N, l.nslices);
+    l.items.num_long = wide ? 0 : shared_items(p, part, N, l.nslices, l.cpl);
     l.items.order = l.items.num_long == part.num_long ? l.items.order : nullptr;
     const int64_t groups =
         l.items.num_long + ((int64_t)part.num_items - l.items.num_long + kWavesPerBlock - 1) / kWavesPerBlock;

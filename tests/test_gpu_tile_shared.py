@@ -38,6 +38,15 @@ def test_shared_items(oracle, N, rows, kind):
     _check(oracle, g, kind, N, rows, dtype="bf16" if N % 2 else "fp16")
 
 
+# Windows of equal length on both sides of the room for four times the waves: 8 rows, N = 128, 2 * 4096 (6.3 steps); 16 rows,
+# N = 128, 0.8 * 4096 (4 steps); 32 rows, N = 128, 0.6 * 3072 (8 steps).  Also items of just under and over 6 steps.
+@pytest.mark.parametrize("rows,windows,degree", [(8, 2040, 26), (8, 2300, 26), (8, 400, 22), (8, 400, 25), (16, 800, 8),
+                                                 (16, 1000, 8), (32, 440, 8), (32, 480, 8)])
+def test_room_for_shared_items(oracle, rows, windows, degree):
+    print(f"[room] rows={rows} windows={windows} degree={degree}", flush=True)
+    _check(oracle, S.random_csr(rows * windows - 3, 1500, degree, seed=rows), 0, 128, rows)
+
+
 def _long_rows(M, K, every, length, seed):
     """Short rows with a long one every `every` rows."""
     rng = np.random.default_rng(seed)
