@@ -77,7 +77,8 @@ __device__ __forceinline__ f32x4 mfma32(u16x8 a, u16x8 b, f32x4 c) {
 // a branch around each the compiler waits for earlier loads in between: 512,000
 // community rows at N = 512 1,215 -> 1,157 us, 64,000 at N = 128 48.3 -> 43.4,
 // 150,000 social rows of 200 at N = 128 769 -> 690, 50,000 of 80 109 -> 91.
-// HalfPointer: 64-bit addresses, for a B of 4 GiB and more.
+// HalfPointer: 64-bit addresses and a branch per gather, for a B of 4 GiB and more
+// and for windows that should stay in step (swept_in_step).
 template <int CPL>
 struct HalfBuffer {
     typedef typename HalfRun<CPL>::T Run;
@@ -831,6 +832,26 @@ TileLaunch tile_launch(const ra_tile_plan* p, const Part& part, const float* C, 
 // B of K rows fits HalfBuffer: the offset of row -1 lies past its end.
 bool half_buffer_fits(int64_t K, int64_t ldb) { return (K + 1) * ldb * 2 <= int64_t{0xFFFFFFFF}; }
 
+// Launches of 8-row windows that keep the branches (HalfPointer): windows in
+// flight together sweep the columns side by side, and the faster their gathers
+// leave the further they drift apart.
+// Windows of about equal length sweep in step by themselves, which shows as soon
+// as the rows of B they sweep (one slice of them where the slices are outermost)
+// pass the 4 MB of an L2 by some; us, buffer / pointers at N = 256: 28,000 rows of
+// 60 75 / 66, 32,000 of 100 135 / 125; at N = 128: 48,000 of 40 45 / 41; but 32,000 of 60
+// at N = 64 (4 MB) 22 / 23; at N = 32: 128,000 of 60 91 / 73, 96,000 (6 MB) 57 / 66.  Shared items have no step to keep.
+// Unequal ones only where the gathers bound the launch: 100,000 rows of 60 at N =
+// 256 32.5 and 34.8 % L2 hits, 357 and 352 us; 250,000 of 500 at N = 512 8,880 and 8,800;
+// 150,000 of 100 at N = 256 880 and 871.  With fewer bytes (50,000 of 80 at N = 128: 91 and
+// 104) or a slice of B that an L2 nearly holds (25,000 of 200 at N = 256: 128 and
+// 140) it is the other way round.
+bool swept_in_step(const ra_tile_plan* p, const Part& part, const TileLaunch& l, int N) {
+    const int64_t slice = static_cast<int64_t>(p->info.K) * std::min(N, 16 * l.cpl) * 2;
+    if (gathered_bytes(p, N) >= kGatherBound && slice > (int64_t{8} << 20)) return true;
+    const int64_t swept = (l.order & 2) ? slice : static_cast<int64_t>(p->info.K) * N * 2;
+    return item_skew(p) < 2 && l.items.num_long < part.num_items && swept >= (l.cpl == 2 ? 7000000 : 8000000);
+}
+
 #define RA_TILE_ARGS                                                                                       \
     l.items, p->atox.get<int32_t>(), p->vals.get<uint16_t>(), Bh, p->info.K, ldb, C, scratch, \
         p->info.M, N, part.num_items, l.nslices, l.order, l.unscale, l.vec_store
@@ -873,18 +894,7 @@ ra_status launch_part(const ra_tile_plan* p, const Part& part, const uint16_t* B
     if (part.num_items == 0) return RA_OK;
     const bool wide = p->info.rows_per_window == 32 && tile_use_mfma32(N);
     const TileLaunch l = tile_launch(p, part, C, scratch, N, wide);
-    // Launches of 8-row windows bound by their gathers keep the branches: windows
-    // in flight together sweep the columns side by side, and the faster their
-    // gathers leave the further they drift apart.  Buffer against pointers:
-    // 100,000 rows of 60 at N = 256 32.5 and 34.8 % L2 hits, 357 and 352 us;
-    // 250,000 of 500 at N = 512 8,880 and 8,800; 150,000 of 100 at N = 256 880 and
-    // 871.  With fewer bytes (50,000 of 80 at N = 128: 91 and 104) or a slice of B that
-    // the 4 MB of an L2 nearly hold (25,000 of 200 at N = 256: 128 and 140) it is the
-    // other way round.
-    const int64_t slice_bytes = static_cast<int64_t>(p->info.K) * std::min(N, 16 * l.cpl) * 2;
-    const bool buf = half_buffer_fits(p->info.K, ldb) &&
-                     !(p->info.rows_per_window == ra::kTileWindow && gathered_bytes(p, N) >= kGatherBound &&
-                       slice_bytes > (int64_t{8} << 20));
+    const bool buf = half_buffer_fits(p->info.K, ldb) && !(p->info.rows_per_window == ra::kTileWindow && swept_in_step(p, part, l, N));
     if (!wide) (buf ? launch_cpl<BF16, HalfBuffer> : launch_cpl<BF16, HalfPointer>)(p, part, l, Bh, ldb, C, scratch, N, st);
     else if (buf) tile_mfma_tall32_kernel<BF16, HalfBuffer<8>><<<l.grid, kBlock, 0, st>>>(RA_TILE_ARGS);
     else tile_mfma_tall32_kernel<BF16, HalfPointer<8>><<<l.grid, kBlock, 0, st>>>(RA_TILE_ARGS);

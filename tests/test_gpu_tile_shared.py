@@ -47,6 +47,15 @@ def test_room_for_shared_items(oracle, rows, windows, degree):
     _check(oracle, S.random_csr(rows * windows - 3, 1500, degree, seed=rows), 0, 128, rows)
 
 
+# Even windows over a B just below and just past the size from which their gathers keep the branches (N = 128: whole rows;
+# N = 512: the slices of TC_DIRECT run outermost; N = 32: narrow runs), fp16 and bf16.
+@pytest.mark.parametrize("K,N", [(31_249, 128), (31_250, 128), (31_250, 512), (62_500, 64), (109_374, 32), (109_375, 32)])
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_even_windows_over_a_large_B(oracle, K, N, kind):
+    print(f"[even] K={K} N={N} kind={kind}", flush=True)
+    _check(oracle, S.random_csr(805, K, 11.0, seed=K % 97), kind, N, 8, dtype="bf16" if kind else "fp16")
+
+
 def _long_rows(M, K, every, length, seed):
     """Short rows with a long one every `every` rows."""
     rng = np.random.default_rng(seed)
