@@ -839,7 +839,8 @@ bool half_buffer_fits(int64_t K, int64_t ldb) { return (K + 1) * ldb * 2 <= int6
 // as the rows of B they sweep (one slice of them where the slices are outermost)
 // pass the 4 MB of an L2 by some; us, buffer / pointers at N = 256: 28,000 rows of
 // 60 75 / 66, 32,000 of 100 135 / 125; at N = 128: 48,000 of 40 45 / 41; but 32,000 of 60
-// at N = 64 (4 MB) 22 / 23; at N = 32: 128,000 of 60 91 / 73, 96,000 (6 MB) 57 / 66.  Shared items have no step to keep.
+// at N = 64 (4 MB) 22 / 23; at N = 32, where short windows and less
+// even ones lose: 128,000 of 60 91 / 73, 144,000 of 12 29 / 34, 96,000 of 60 (6 MB) 57 / 66.  Shared items have no step to keep.
 // Unequal ones only where the gathers bound the launch: 100,000 rows of 60 at N =
 // 256 32.5 and 34.8 % L2 hits, 357 and 352 us; 250,000 of 500 at N = 512 8,880 and 8,800;
 // 150,000 of 100 at N = 256 880 and 871.  With fewer bytes (50,000 of 80 at N = 128: 91 and
@@ -849,7 +850,9 @@ bool swept_in_step(const ra_tile_plan* p, const Part& part, const TileLaunch& l,
     const int64_t slice = static_cast<int64_t>(p->info.K) * std::min(N, 16 * l.cpl) * 2;
     if (gathered_bytes(p, N) >= kGatherBound && slice > (int64_t{8} << 20)) return true;
     const int64_t swept = (l.order & 2) ? slice : static_cast<int64_t>(p->info.K) * N * 2;
-    return item_skew(p) < 2 && l.items.num_long < part.num_items && swept >= (l.cpl == 2 ? 7000000 : 8000000);
+    if (l.items.num_long >= part.num_items) return false;
+    if (l.cpl == 2) return item_skew(p) < 1.5 && p->info.num_blocks >= 28LL * p->num_items && swept >= 7000000;
+    return item_skew(p) < 2 && swept >= 8000000;
 }
 
 #define RA_TILE_ARGS                                                                                       \

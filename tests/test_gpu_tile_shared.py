@@ -53,7 +53,7 @@ def test_room_for_shared_items(oracle, rows, windows, degree):
 @pytest.mark.parametrize("kind", [0, 1, 2])
 def test_even_windows_over_a_large_B(oracle, K, N, kind):
     print(f"[even] K={K} N={N} kind={kind}", flush=True)
-    _check(oracle, S.random_csr(805, K, 11.0, seed=K % 97), kind, N, 8, dtype="bf16" if kind else "fp16")
+    _check(oracle, S.random_csr(805, K, 32.0 if N == 32 else 11.0, seed=K % 97), kind, N, 8, dtype="bf16" if kind else "fp16")
 
 
 def _long_rows(M, K, every, length, seed):
