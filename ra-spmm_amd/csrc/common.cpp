@@ -54,7 +54,10 @@ struct PoolBlock {
 
 struct DevicePool {
     std::multimap<size_t, PoolBlock> free_blocks;  // by capacity
-    size_t held = 0;
+    // Given back while the device may still be using them: free once it has
+    // been waited for, which the first request that could use one does.
+    std::multimap<size_t, PoolBlock> pending;
+    size_t held = 0;  // bytes of both
 };
 
 struct Pool {
@@ -70,8 +73,9 @@ Pool& pool() {
     return *p;
 }
 
-// Eight classes per power of two: at most 1/8 is wasted, and plans of graphs of
-// about the same size use each other's blocks.
+// Eight classes per power of two, so that plans of graphs of about the same size
+// use each other's blocks; a class is at most 1/8 over the request, and a kept
+// block at most 1/4 over its class (take). 
 size_t size_class(size_t bytes) {
     size_t power = 4096;
     while (power * 2 <= bytes) power *= 2;
@@ -96,71 +100,102 @@ private:
     bool switched_ = false;
 };
 
-// Free the blocks of `d` from the oldest on until at most `keep` bytes are held.
+// hipFree, which waits for the device by itself.  Its error (a stream is being
+// captured) is not left for the next launch check.
+bool free_block(void* ptr) {
+    if (hipFree(ptr) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
+// Free the blocks of `d` from the oldest on until at most `keep` bytes are held,
+// or until one cannot be freed now.
 void trim_locked(int device, DevicePool& d, size_t keep) {
     if (d.held <= keep) return;
     const OnDevice on(device);
-    while (d.held > keep && !d.free_blocks.empty()) {
-        auto oldest = d.free_blocks.begin();
-        for (auto it = d.free_blocks.begin(); it != d.free_blocks.end(); ++it)
-            if (it->second.age < oldest->second.age) oldest = it;
-        (void)hipFree(oldest->second.ptr);
+    while (d.held > keep) {
+        std::multimap<size_t, PoolBlock>* list = nullptr;
+        std::multimap<size_t, PoolBlock>::iterator oldest;
+        for (auto* l : {&d.free_blocks, &d.pending})
+            for (auto it = l->begin(); it != l->end(); ++it)
+                if (!list || it->second.age < oldest->second.age) {
+                    list = l;
+                    oldest = it;
+                }
+        if (!list || !free_block(oldest->second.ptr)) return;
         d.held -= oldest->first;
-        d.free_blocks.erase(oldest);
+        list->erase(oldest);
     }
+}
+
+// A kept block of `want` bytes or a quarter more, or the end of the list.
+std::multimap<size_t, PoolBlock>::iterator find_block(std::multimap<size_t, PoolBlock>& list, size_t want) {
+    const auto it = list.lower_bound(want);
+    return it != list.end() && it->first <= want + want / 4 ? it : list.end();
+}
+
+bool take(DevicePool& d, size_t want, void** ptr, size_t* capacity) {
+    const auto it = find_block(d.free_blocks, want);
+    if (it == d.free_blocks.end()) return false;
+    *ptr = it->second.ptr;
+    *capacity = it->first;
+    d.held -= it->first;
+    d.free_blocks.erase(it);
+    return true;
 }
 
 }  // namespace
 
-ra_status pool_allocate(void** ptr, size_t bytes, size_t* capacity, int* device) {
+ra_status pool_allocate(void** ptr, size_t bytes, bool kept, size_t* capacity, int* device) {
     *ptr = nullptr;
     RA_HIP_TRY(hipGetDevice(device));
-    const size_t want = size_class(bytes);
+    const size_t want = kept ? size_class(bytes) : bytes;
     Pool& p = pool();
-    {
-        std::lock_guard<std::mutex> lock(p.mutex);
-        DevicePool& d = p.devices[*device];
-        const auto it = d.free_blocks.lower_bound(want);
-        if (it != d.free_blocks.end() && it->first <= want + want / 4) {
-            *ptr = it->second.ptr;
-            *capacity = it->first;
-            d.held -= it->first;
-            d.free_blocks.erase(it);
-            return RA_OK;
+    if (kept) {
+        std::multimap<size_t, PoolBlock> waited;
+        {
+            std::lock_guard<std::mutex> lock(p.mutex);
+            DevicePool& d = p.devices[*device];
+            if (take(d, want, ptr, capacity)) return RA_OK;
+            if (find_block(d.pending, want) != d.pending.end()) waited.swap(d.pending);
+        }
+        if (!waited.empty()) {
+            const bool idle = hipDeviceSynchronize() == hipSuccess;
+            if (!idle) (void)hipGetLastError();  // a stream is being captured: they stay pending
+            std::lock_guard<std::mutex> lock(p.mutex);
+            DevicePool& d = p.devices[*device];
+            (idle ? d.free_blocks : d.pending).merge(waited);
+            if (idle && take(d, want, ptr, capacity)) return RA_OK;
         }
     }
-    hipError_t e = hipMalloc(ptr, want);
+    size_t size = want;
+    hipError_t e = hipMalloc(ptr, size);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
         {
             std::lock_guard<std::mutex> lock(p.mutex);
             trim_locked(*device, p.devices[*device], 0);
         }
-        e = hipMalloc(ptr, want);
+        e = hipMalloc(ptr, size);
     }
     if (e != hipSuccess) {
         *ptr = nullptr;
         return hip_fail(e, "hipMalloc");
     }
-    *capacity = want;
+    *capacity = size;
     return RA_OK;
 }
 
 void pool_release(void* ptr, size_t capacity, int device, bool idle) {
-    {
-        // What cannot be waited for (a stream of this thread is being captured)
-        // is not reused.
+    if (capacity > kPoolBytes) {
         const OnDevice on(device);
-        if (capacity > kPoolBytes || (!idle && hipDeviceSynchronize() != hipSuccess)) {
-            (void)hipGetLastError();
-            (void)hipFree(ptr);
-            return;
-        }
+        (void)free_block(ptr);
+        return;
     }
     Pool& p = pool();
     std::lock_guard<std::mutex> lock(p.mutex);
     DevicePool& d = p.devices[device];
-    d.free_blocks.emplace(capacity, PoolBlock{ptr, ++p.clock});
+    (idle ? d.free_blocks : d.pending).emplace(capacity, PoolBlock{ptr, ++p.clock});
     d.held += capacity;
     trim_locked(device, d, kPoolBytes);
 }

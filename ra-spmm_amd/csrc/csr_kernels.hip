@@ -910,7 +910,7 @@ static ra_status zo_run(ra_zo_plan* plan, const int32_t* d_rowptr, const int32_t
     const int zslice = tuning().zo_slice >= 0 ? tuning().zo_slice : vec ? column_slice(load, 0) : 0;
     LaneShape sh = pick_shape(np, vec ? 4 : 1, zslice);
     if (plan->info.num_split_chunks > 0 && !partials) {
-        RA_TRY(plan->partials.ensure((size_t)plan->info.num_split_chunks * N * sizeof(float)));
+        RA_TRY(plan->partials.ensure((size_t)plan->info.num_split_chunks * N * sizeof(float), st));
         partials = plan->partials.get<float>();
     }
     const int RPW = kWave / sh.G;

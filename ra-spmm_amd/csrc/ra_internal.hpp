@@ -55,13 +55,15 @@ inline ra_status hip_fail(hipError_t e, const char* what) {
 // GB for 512,000 rows and 1.6e7 nonzeros) cost a one-off call 10 to 40 ms
 // against 3 ms of kernels; from the pool they cost nothing.
 //
-// Streams and threads: a block enters the pool only once nothing on the device
-// can still be using it, as hipFree would wait for (`idle` says that the caller
-// has waited already), so the next owner may use it on any stream.  The lists
-// are locked.  Memory goes back to the driver when the pool is full (oldest
+// Streams and threads: a block is handed on only once the device has been waited
+// for after it was given back (`idle`: the caller has waited already), so the
+// next owner may use it on any stream.  Giving back calls nothing that a stream
+// capture forbids, unless the pool is full or the block is larger than it.  The
+// lists are locked.  Memory goes back to the driver when the pool is full (oldest
 // block first), when an allocation fails, and on pool_trim().
+// kept = false: straight from the driver.
 constexpr size_t kPoolBytes = size_t(4) << 30;
-ra_status pool_allocate(void** ptr, size_t bytes, size_t* capacity, int* device);
+ra_status pool_allocate(void** ptr, size_t bytes, bool kept, size_t* capacity, int* device);
 void pool_release(void* ptr, size_t capacity, int device, bool idle);
 void pool_trim();
 
@@ -86,7 +88,7 @@ public:
         return *this;
     }
 
-    ra_status allocate(size_t bytes) {
+    ra_status allocate(size_t bytes, bool kept = true) {
         reset();
         if (bytes == 0) return RA_OK;
         // RA_MAX_ALLOC_BYTES caps one allocation (read per call): a larger one
@@ -97,12 +99,16 @@ public:
                 return fail(RA_ERR_OUT_OF_MEMORY, "hipMalloc: " + std::to_string(bytes) +
                                                       " bytes exceed RA_MAX_ALLOC_BYTES");
         }
-        return pool_allocate(&ptr_, bytes, &bytes_, &device_);
+        return pool_allocate(&ptr_, bytes, kept, &bytes_, &device_);
     }
-    // Grow-only reuse (plan scratch).
-    ra_status ensure(size_t bytes) {
+    // Grow-only reuse (plan scratch) for work on `stream`.  While that is being
+    // captured the driver decides: it refuses, and the run that sizes the scratch
+    // has to come before the capture whatever the pool holds.
+    ra_status ensure(size_t bytes, hipStream_t stream) {
         if (bytes <= bytes_) return RA_OK;
-        return allocate(bytes);
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
+        return allocate(bytes, capture == hipStreamCaptureStatusNone);
     }
     template <typename T>
     ra_status upload(const std::vector<T>& v) {

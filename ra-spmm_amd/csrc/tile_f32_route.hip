@@ -197,7 +197,7 @@ ra_status tile_f32_prepare(ra_tile_plan* p, hipStream_t st) {
         RA_HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, sb, keys.get<uint64_t>(), keys2.get<uint64_t>(),
                                                       v1.get<float>(), p->f32_vals.get<float>(),
                                                       static_cast<int>(n), 0, cb + rbits, st));
-        RA_TRY(tmp.ensure(std::max<size_t>(sb, 1)));
+        RA_TRY(tmp.ensure(std::max<size_t>(sb, 1), st));
         RA_HIP_TRY(hipcub::DeviceRadixSort::SortPairs(tmp.get(), sb, keys.get<uint64_t>(), keys2.get<uint64_t>(),
                                                       v1.get<float>(), p->f32_vals.get<float>(),
                                                       static_cast<int>(n), 0, cb + rbits, st));
@@ -212,7 +212,7 @@ ra_status tile_f32_prepare(ra_tile_plan* p, hipStream_t st) {
         size_t ms = 0;
         RA_HIP_TRY(hipcub::DeviceScan::InclusiveScan(nullptr, ms, last.get<int32_t>(), rowptr + 1, hipcub::Max(),
                                                      static_cast<int>(R), st));
-        RA_TRY(tmp.ensure(std::max<size_t>(ms, 1)));
+        RA_TRY(tmp.ensure(std::max<size_t>(ms, 1), st));
         RA_HIP_TRY(hipcub::DeviceScan::InclusiveScan(tmp.get(), ms, last.get<int32_t>(), rowptr + 1, hipcub::Max(),
                                                      static_cast<int>(R), st));
         RA_HIP_TRY(hipStreamSynchronize(st));  // before `last`, `keys*`, `v1` and `tmp` are freed

@@ -924,7 +924,7 @@ ra_status launch_merge(const ra_tile_plan* p, const Part& part, float* C, int N,
 ra_status run_common(ra_tile_plan* p, const uint16_t* Bh, int ldb, bool bf16, float* C, int N, hipStream_t st) {
     float* scratch = nullptr;
     if (p->info.num_split_segs > 0) {
-        RA_TRY(p->scratch.ensure((size_t)p->info.num_split_segs * p->info.rows_per_window * N * sizeof(float)));
+        RA_TRY(p->scratch.ensure((size_t)p->info.num_split_segs * p->info.rows_per_window * N * sizeof(float), st));
         scratch = p->scratch.get<float>();
     }
     // Column partitions run one after another on the stream, each adding into
@@ -1019,7 +1019,7 @@ ra_status ra_tile_plan_run(ra_tile_plan* p, const float* d_B, float* d_C, int32_
     if (bf16 != (p->info.value_dtype == RA_DTYPE_BF16))
         return ra::fail(RA_ERR_INVALID_ARGUMENT, "tile: route precision differs from the plan's value dtype");
     const int ldb = (N + 7) / 8 * 8;
-    RA_TRY(p->bconv.ensure((size_t)p->info.K * ldb * sizeof(uint16_t)));
+    RA_TRY(p->bconv.ensure((size_t)p->info.K * ldb * sizeof(uint16_t), st));
     RA_TRY(launch_convert(d_B, p->bconv.get(), p->info.K, N, ldb, bf16, st));
     return run_common(p, p->bconv.get<uint16_t>(), ldb, bf16, d_C, N, st);
 }

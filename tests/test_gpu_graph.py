@@ -3,6 +3,8 @@ then), captured into a HIP graph through torch.cuda.graph, and replayed several
 times with eager work and synchronisations in between.  Each replay must equal
 the eager result bit for bit (the kernels are deterministic and no path records
 a memset into the graph)."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -41,3 +43,40 @@ def test_capture_and_replay(label, N):
         torch.cuda.synchronize()
         assert torch.equal(out, eager), (label, i)
         del junk
+
+
+def _capture(fn):
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = fn()
+    return graph, out
+
+
+def test_plan_dropped_during_a_capture():
+    """Giving a plan back, on the capturing thread or another, neither ends a capture nor hands its memory on before the
+    work queued with it is done."""
+    g = S.random_csr(3000, 2500, 14.0, seed=7, skew=0.9, max_deg=1500)
+    rp, ci, vl = g.torch("cuda")
+    B = torch.randn(g.K, 96, device="cuda")
+    run = lambda p: ra_spmm.run_segment_hybrid_plan(p, ci, vl, B)  # noqa: E731
+    plans = [ra_spmm.make_segment_hybrid_plan(rp, ci, vl, g.M, g.K, 96) for _ in range(3)]
+    want = [run(p) for p in plans][0]
+    torch.cuda.synchronize()
+
+    def body():
+        first = run(plans[0])
+        del plans[2]
+        other = threading.Thread(target=plans.pop)
+        other.start()
+        other.join()
+        return first, run(plans[0])
+
+    graph, outs = _capture(body)
+    assert len(plans) == 1
+    for _ in range(3):
+        new = ra_spmm.make_segment_hybrid_plan(rp, ci, vl, g.M, g.K, 96)  # takes the dropped plans' memory
+        assert torch.equal(run(new), want)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, want) for o in outs)
+        del new
