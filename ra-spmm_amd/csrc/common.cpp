@@ -75,8 +75,10 @@ Pool& pool() {
 
 // Eight classes per power of two, so that plans of graphs of about the same size
 // use each other's blocks; a class is at most 1/8 over the request, and a kept
-// block at most 1/4 over its class (take). 
+// block at most 1/4 over its class (take).  What the pool never keeps is not
+// rounded.
 size_t size_class(size_t bytes) {
+    if (bytes > kPoolBytes) return bytes;
     size_t power = 4096;
     while (power * 2 <= bytes) power *= 2;
     const size_t step = power / 8;
@@ -176,6 +178,7 @@ ra_status pool_allocate(void** ptr, size_t bytes, bool kept, size_t* capacity, i
             std::lock_guard<std::mutex> lock(p.mutex);
             trim_locked(*device, p.devices[*device], 0);
         }
+        size = bytes;  // no more than was asked for
         e = hipMalloc(ptr, size);
     }
     if (e != hipSuccess) {

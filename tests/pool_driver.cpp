@@ -119,6 +119,16 @@ int main() {
     }
     ra::pool_trim();
     CHECK(total == 0);
+    {  // Sizes: rounded up by an eighth at most, not where the pool would not keep it or nothing else fits.
+        DeviceBuffer a;
+        CHECK(a.allocate(1000 * kMiB + 1) == RA_OK && last_size > 1000 * kMiB && last_size <= 1125 * kMiB + 1);
+        CHECK(a.allocate(5 * kGiB + 4096) == RA_OK && last_size == 5 * kGiB + 4096);
+        a.reset();
+        limit = 3 * kGiB + 64 * kMiB;
+        CHECK(a.allocate(3 * kGiB + 32 * kMiB) == RA_OK && last_size == 3 * kGiB + 32 * kMiB && a.bytes() == last_size);
+        CHECK(a.allocate(3 * kGiB + 65 * kMiB) == RA_ERR_OUT_OF_MEMORY && a.get() == nullptr && a.bytes() == 0);
+        CHECK(a.allocate(3 * kGiB) == RA_OK);
+    }
     std::printf("pool ok\n");
     return 0;
 }

@@ -40,6 +40,34 @@ def test_reuse_and_release():
     assert torch.equal(once(), ref)
 
 
+def test_bound_and_large_blocks():
+    """Dropped plans keep at most 4 GiB, and a block above that takes what was asked for and goes back at once."""
+    ra_spmm.release_memory()
+    g = S.random_csr(4096, 600_000, 4.0, seed=3)
+    rp, ci, vl = g.torch("cuda")
+
+    def run(n):
+        plan = ra_spmm.make_tc_direct_plan(rp, ci, vl, g.M, g.K, n)
+        ra_spmm.run_tc_direct_plan(plan, torch.zeros(g.K, n, device="cuda"))
+        torch.cuda.synchronize()
+        return plan
+
+    run(64)
+    ra_spmm.release_memory()
+    start = _free()
+    plans = [run(1024) for _ in range(5)]  # 1.2 GB each
+    assert start - _free() > 5 * g.K * 1024 * 2
+    plans.clear()
+    assert start - _free() < (4 << 30) + (64 << 20)
+    ra_spmm.release_memory()
+    assert start - _free() < (64 << 20)
+    plan = run(3712)  # 4.45 GB: eighths of its power of two would be 4.83
+    need = g.K * 3712 * 2
+    assert abs(start - _free() - need) < (256 << 20)  # the runtime's own memory comes and goes by some MiB
+    del plan
+    assert start - _free() < (256 << 20)
+
+
 def test_plans_of_other_streams_and_threads():
     """A plan dropped right after its run was queued on a side stream: the next plans, on other streams and threads,
     must not get its memory before the run is done."""
