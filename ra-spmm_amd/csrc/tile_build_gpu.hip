@@ -697,9 +697,11 @@ ra_status gpu_build(ra_tile_plan* p, int32_t kind, const int32_t* rowptr, const 
     float vmax;
     std::memcpy(&vmax, &hflags[2], 4);
     // Rows in order, one column range, every window of 32 rows in one
-    // workgroup's LDS and its keys in 32 bits: windows are sorted there.
+    // workgroup's LDS and its keys in 32 bits: windows are sorted there, a
+    // workgroup each (a grid holds 2^32 work-items: 134 million rows).
     const int longest = static_cast<int>(hflags[3]);
-    const bool sort_windows = kind != RA_TILE_COMMUNITY_TC && P == 1 && longest <= kWindowSortMax && cb + 5 <= 32;
+    const bool sort_windows = kind != RA_TILE_COMMUNITY_TC && P == 1 && longest <= kWindowSortMax && cb + 5 <= 32 &&
+                              (static_cast<int64_t>(M) + ra::kTileWindow - 1) / ra::kTileWindow * kThreads <= UINT32_MAX;
     p->info.value_scale_log2 = bf16 ? 0 : ra::f16_value_scale_log2(vmax);
     const float vscale = std::ldexp(1.0f, p->info.value_scale_log2);
 

@@ -152,3 +152,28 @@ def test_window_height_choice(longest):
             2.0 ** -25 * ra_spmm.spmm_csr_baseline(rp, ci, vl.abs(), torch.ones_like(B)) + 1e-30
         for p in plans:
             assert bool(((ra_spmm.run_tile_plan_route(p, B, "fp16") - ref).abs() <= bound).all())
+
+
+def test_more_windows_than_a_grid():
+    """134 million rows: more 8-row windows than one workgroup each would fit a grid."""
+    if torch.cuda.get_device_properties(0).total_memory < 64 << 30:
+        pytest.skip("needs a GPU with 64 GiB")
+    M, K, N = (1 << 27) + 11, 500, 16
+    print(f"[windows] M={M}", flush=True)
+    rows = torch.cat([torch.arange(300), torch.arange(1 << 26, (1 << 26) + 300), torch.arange(M - 300, M)])
+    deg = torch.zeros(M, dtype=torch.int32, device="cuda")
+    deg[rows.cuda()] = 7
+    rowptr = torch.zeros(M + 1, dtype=torch.int32, device="cuda")
+    rowptr[1:] = torch.cumsum(deg, 0)
+    gen = torch.Generator("cuda").manual_seed(1)
+    ci = torch.sort(torch.rand(rows.numel(), K, device="cuda", generator=gen).topk(7, dim=1).indices, dim=1).values
+    ci = ci.to(torch.int32).flatten()
+    vl = torch.randint(1, 65, (ci.numel(),), device="cuda", generator=gen) / 64.0
+    B = torch.randn(K, N, device="cuda", generator=gen).half().float()
+    plan = ra_spmm.make_tc_direct_plan(rowptr, ci, vl, M, K, N)
+    assert plan.nnz == ci.numel() and plan.num_windows == (M + 7) // 8
+    C = ra_spmm.run_tc_direct_plan(plan, B)
+    want = (vl.double()[:, None] * B.double()[ci.long()]).view(-1, 7, N).sum(1)
+    scale = (vl.double()[:, None] * B.double().abs()[ci.long()]).view(-1, 7, N).sum(1)
+    assert ((C[rows.cuda()].double() - want).abs() <= 1e-5 * scale).all()
+    assert int((C != 0).any(1).sum()) <= rows.numel()
