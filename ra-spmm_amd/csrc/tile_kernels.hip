@@ -580,7 +580,9 @@ __global__ __launch_bounds__(kBlock, 2) void tile_mfma_tall32_kernel(
 // C[w*8+m][n] = ((slot0 + slot1) + ...) in ascending slot order
 // (tc/ra_segment_hybrid.cu:198-221).  A thread owns one column of one window
 // row and loads kDeep slots at a time, so a long window's chain is its additions
-// and not a memory latency per slot.
+// and not a memory latency per slot.  Index: 32 bits where the window's H * N
+// elements and the last step of the grid fit them.
+template <typename Index>
 __global__ __launch_bounds__(kBlock) void tile_merge_kernel(
     const int32_t* __restrict__ split_windows, const int32_t* __restrict__ split_offsets,
     const int32_t* __restrict__ win_rows, const float* __restrict__ scratch, float* __restrict__ C,
@@ -589,10 +591,10 @@ __global__ __launch_bounds__(kBlock) void tile_merge_kernel(
     const int sw = blockIdx.x;
     const int o0 = split_offsets[sw], o1 = split_offsets[sw + 1];
     const int64_t window = split_windows[sw] - cell_base;
-    const uint32_t count = static_cast<uint32_t>(H) * N;
+    const Index count = static_cast<Index>(H) * N;
     // grid.y is capped by the launch; stride over the window's H*N elements.
-    for (uint32_t e = blockIdx.y * kBlock + threadIdx.x; e < count; e += gridDim.y * kBlock) {
-        const uint32_t m = e / static_cast<uint32_t>(N);
+    for (Index e = blockIdx.y * kBlock + threadIdx.x; e < count; e += gridDim.y * kBlock) {
+        const uint32_t m = static_cast<uint32_t>(e / static_cast<Index>(N));
         const int64_t slot_row = window * H + m;
         const int row = win_rows ? win_rows[slot_row] : static_cast<int>(slot_row);
         if (row < 0 || row >= M) continue;
@@ -607,7 +609,7 @@ __global__ __launch_bounds__(kBlock) void tile_merge_kernel(
             for (int k = 0; k < kDeep; ++k) acc += x[k];
         }
         for (; o < o1; ++o) acc += part[(int64_t)o * count];
-        float* dst = C + (int64_t)row * N + (e - m * N);
+        float* dst = C + (int64_t)row * N + (e - static_cast<Index>(m) * N);
         *dst = accumulate ? *dst + acc : acc;
     }
 }
@@ -912,10 +914,10 @@ ra_status launch_merge(const ra_tile_plan* p, const Part& part, float* C, int N,
     dim3 grid(part.num_splits,
               static_cast<unsigned>(std::min<int64_t>(((int64_t)H * N + kBlock - 1) / kBlock, 65535)));
     const int32_t* wr = p->info.kind == RA_TILE_COMMUNITY_TC ? p->win_rows.get<int32_t>() : nullptr;
-    tile_merge_kernel<<<grid, kBlock, 0, st>>>(p->split_windows.get<int32_t>() + part.split_base,
-                                               p->split_offsets.get<int32_t>() + part.split_base, wr,
-                                               p->scratch.get<float>(), C, p->info.M, N, H, part.cell_base,
-                                               part.accumulate);
+    const bool small = static_cast<int64_t>(H) * N + 65535LL * kBlock <= int64_t{0xFFFFFFFF};
+    (small ? tile_merge_kernel<uint32_t> : tile_merge_kernel<int64_t>)<<<grid, kBlock, 0, st>>>(
+        p->split_windows.get<int32_t>() + part.split_base, p->split_offsets.get<int32_t>() + part.split_base, wr,
+        p->scratch.get<float>(), C, p->info.M, N, H, part.cell_base, part.accumulate);
     RA_LAUNCH_CHECK("tile_merge_kernel");
     return RA_OK;
 }
