@@ -1014,8 +1014,13 @@ ra_status ra_tile_plan_create_device(int32_t kind, const int32_t* d_rowptr, cons
         delete p;
         return ra::fail(RA_ERR_INVALID_ARGUMENT, "tile: rows_per_window must be 0 (auto), 8, 16 or 32");
     }
-    const ra_status s = gpu_build(p, kind, d_rowptr, d_colind, d_vals, M, K, N, value_dtype, rows_per_window,
-                                  reinterpret_cast<hipStream_t>(stream));
+    ra_status s;
+    try {
+        s = gpu_build(p, kind, d_rowptr, d_colind, d_vals, M, K, N, value_dtype, rows_per_window,
+                      reinterpret_cast<hipStream_t>(stream));
+    } catch (const std::bad_alloc&) {
+        s = ra::fail(RA_ERR_OUT_OF_MEMORY, "tile: host memory of the build");
+    }
     if (s != RA_OK) {
         delete p;
         return s;

@@ -986,15 +986,21 @@ ra_status ra_tile_plan_create(int32_t kind, const int32_t* h_rowptr, const int32
             (s = p->split_windows.upload(host.split_windows)) == RA_OK &&
             (s = p->split_offsets.upload(host.split_offsets)) == RA_OK) {
             p->num_items = p->info.num_segments;
-            std::vector<int32_t> order;
-            for (int pass = 0; pass < 2; ++pass)
-                for (int32_t i = 0; i < p->num_items; ++i)
-                    if ((host.seg_bend[i] - host.seg_bbegin[i] > ra::kTileLongBlocks) == (pass == 0)) {
-                        order.push_back(i);
-                        p->part_long[0] += pass == 0;
-                    }
+            auto is_long = [&](int32_t i) { return host.seg_bend[i] - host.seg_bbegin[i] > ra::kTileLongBlocks; };
+            for (int32_t i = 0; i < p->num_items; ++i) p->part_long[0] += is_long(i);
             p->has_long = p->part_long[0] > 0;
-            s = p->item_order.upload(order);
+            if (p->has_long) {
+                try {
+                    std::vector<int32_t> order;
+                    order.reserve(p->num_items);
+                    for (int pass = 0; pass < 2; ++pass)
+                        for (int32_t i = 0; i < p->num_items; ++i)
+                            if (is_long(i) == (pass == 0)) order.push_back(i);
+                    s = p->item_order.upload(order);
+                } catch (const std::bad_alloc&) {
+                    s = ra::fail(RA_ERR_OUT_OF_MEMORY, "tile: host build out of memory");
+                }
+            }
         }
     }
     if (s != RA_OK) {
