@@ -394,17 +394,29 @@ def bench_config(cfg, N, steps, warmup, table, do_cpu, cold_reps=10, force_path=
     ra_spmm.run_planned_kernel(label, warm_plan, rp, ci, vl, B)
     del warm_plan
     torch.cuda.synchronize()
-    build_ms, first_ms = [], []
-    for _ in range(cold_reps):
-        torch.cuda.synchronize()
-        t = time.perf_counter()
-        plan = ra_spmm.build_kernel_plan(label, rp_cpu, ci_cpu, vl_cpu, g.M, g.K, N)
-        torch.cuda.synchronize()
-        build_ms.append((time.perf_counter() - t) * 1e3)
-        out, ms = ra_spmm.measure_one_ms(lambda: ra_spmm.run_planned_kernel(label, plan, rp, ci, vl, B))
-        first_ms.append(ms)
-        del out, plan
-        torch.cuda.synchronize()
+
+    def cold_builds(keep_memory):
+        """Mean ms of build and first execution; unless keep_memory, every repetition allocates from the driver, as a
+        process's first plan and rocSPARSE's timed call do."""
+        build, first = [], []
+        for _ in range(cold_reps):
+            if not keep_memory:
+                ra_spmm.release_memory()
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            plan = ra_spmm.build_kernel_plan(label, rp_cpu, ci_cpu, vl_cpu, g.M, g.K, N)
+            torch.cuda.synchronize()
+            build.append((time.perf_counter() - t) * 1e3)
+            out, ms = ra_spmm.measure_one_ms(lambda: ra_spmm.run_planned_kernel(label, plan, rp, ci, vl, B))
+            first.append(ms)
+            del out, plan
+            torch.cuda.synchronize()
+        return sum(build) / cold_reps, sum(first) / cold_reps
+
+    kept = cold_builds(True)
+    build_ms, first_ms = cold_builds(False)
+    log(f"[bench] cold build {build_ms:.3f} ms, first execution {first_ms:.3f} ms; with the memory of earlier plans "
+        f"{kept[0]:.3f} and {kept[1]:.3f}")
     plan = ra_spmm.build_kernel_plan(label, rp_cpu, ci_cpu, vl_cpu, g.M, g.K, N)
 
     run = lambda: ra_spmm.run_planned_kernel(label, plan, rp, ci, vl, B)  # noqa: E731
@@ -437,8 +449,8 @@ def bench_config(cfg, N, steps, warmup, table, do_cpu, cold_reps=10, force_path=
         "kernel": k_name, "kernel_ms": k_ms, "bytes_alg": b_alg,
         "bytes_edgewise": bytes_edgewise(g.M, g.nnz, N),
         "cold_route_ms": sum(route_ms) / len(route_ms),
-        "cold_build_ms": sum(build_ms) / len(build_ms),
-        "cold_first_exec_ms": sum(first_ms) / len(first_ms),
+        "cold_build_ms": build_ms,
+        "cold_first_exec_ms": first_ms,
         "baseline_ms": base_wall, "baseline_gflops": flops / (base_wall * 1e-3) / 1e9,
         "csr_direct_ms": cd_wall, "csr_direct_gflops": flops / (cd_wall * 1e-3) / 1e9,
         "speedup_vs_baseline": base_wall / wall_ms,
@@ -453,17 +465,25 @@ def bench_config(cfg, N, steps, warmup, table, do_cpu, cold_reps=10, force_path=
     # experiments/deployed_coldstart.py): device feature pass + route, then a
     # path without a tile-format build, every overhead in, device CSR.
     ra_spmm.run_deployed_cold(rp, ci, vl, B, table)  # untimed: code objects
-    dts = []
-    for _ in range(cold_reps):
-        torch.cuda.synchronize()
-        t = time.perf_counter()
-        out_d, dlab = ra_spmm.run_deployed_cold(rp, ci, vl, B, table)
-        torch.cuda.synchronize()
-        dts.append((time.perf_counter() - t) * 1e3)
-        del out_d
-    res["deployed_cold"] = {"path": dlab, "ms": sum(dts) / len(dts),
-                            "speedup_vs_rocsparse": (roc["cold_ms"] / (sum(dts) / len(dts)))
-                            if roc.get("cold_ms") else None}
+
+    def deployed(keep_memory):
+        total = 0.0
+        for _ in range(cold_reps):
+            if not keep_memory:
+                ra_spmm.release_memory()
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            out_d, path = ra_spmm.run_deployed_cold(rp, ci, vl, B, table)
+            torch.cuda.synchronize()
+            total += (time.perf_counter() - t) * 1e3
+            del out_d
+        return total / cold_reps, path
+
+    kept_ms, _ = deployed(True)
+    deployed_ms, dlab = deployed(False)
+    log(f"[bench] deployed cold call {deployed_ms:.4f} ms; with the memory of earlier plans {kept_ms:.4f}")
+    res["deployed_cold"] = {"path": dlab, "ms": deployed_ms,
+                            "speedup_vs_rocsparse": roc["cold_ms"] / deployed_ms if roc.get("cold_ms") else None}
     cold_total = res["cold_route_ms"] + res["cold_build_ms"] + res["cold_first_exec_ms"]
     res["cold_total_ms"] = cold_total
     res["cold_speedup_vs_rocsparse"] = (roc["cold_ms"] / cold_total) if roc.get("cold_ms") else None
