@@ -31,7 +31,8 @@ extern "C" {
 #define RA_SPMM_ABI_VERSION 1
 
 /* Plan and scratch memory of destroyed plans is kept for the next ones, up to
- * 4 GiB per device; this gives all of it back to the driver. */
+ * 4 GiB per device; this gives all of it back to the driver.  Other allocators
+ * of the process cannot reclaim it. */
 void ra_release_memory(void);
 
 /* Opaque stream handle: identical to hipStream_t (struct ihipStream_t*). */

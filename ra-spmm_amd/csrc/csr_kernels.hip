@@ -713,19 +713,19 @@ struct RowLoad {
 // of the waves, lane permutes and instructions, but their loads straddle cache
 // sectors, so one a lane wins where the gathered bytes set the time and where
 // four would leave a group's lanes unused.  us, four / one:
-//   N <= 8: always.  300,000 rows of 20 at N = 5 63 / 51; hubs, 20,000 rows of 12
+//   N <= 8: always.  300,000 rows of 20 at N = 5 85 / 65; hubs, 20,000 rows of 12
 //   16 / 10.
 //   N <= 16: unless rows are short, where waves count: 100,000 rows of 3 at N = 13
-//   8.5 / 10.8, 50,000 of 6 5.1 / 5.8, 300,000 of 20 107 / 86; hubs, 1e6 rows of 12
-//   257 / 238.
+//   6.7 / 8.5, 50,000 of 6 5.1 / 5.8, 300,000 of 20 144 / 121; hubs, 1e6 rows of 12
+//   278 / 255.
 //   N <= 32 with hub rows, whose chains get 16 gathers in flight instead of 8, or
-//   long rows: hubs, 20,000 rows of 24 at N = 30 24 / 17, 200,000 of 6 38 / 43.
+//   long rows: hubs, 20,000 rows of 24 at N = 30 19 / 14, 200,000 of 6 42 / 48.
 //   N <= 128 where a one-column wave gathers 3,000 bytes (2,000 from a large B of
-//   narrow rows) and B is well past the L2s: 300,000 rows of 32 at N = 30 378 / 342, of
-//   8 at N = 33 94 / 110; 30,000 of 20 at N = 33 13 / 18; 50,000 uneven rows of 15 at
+//   narrow rows) and B is well past the L2s: 300,000 rows of 32 at N = 30 325 / 297, of
+//   8 at N = 33 85 / 100; 30,000 of 20 at N = 33 12 / 18; 50,000 uneven rows of 15 at
 //   N = 65 55 / 69.
-//   Wider, both take the same time (100,000 rows of 20 at N = 225 229 / 229) or
-//   four win (20,000 rows of 12 with hubs 28 / 38).
+//   Wider, both take the same time (100,000 rows of 20 at N = 225 285 / 285) or
+//   four win (20,000 rows of 12 with hubs 30 / 40).
 inline bool one_column_packets(const RowLoad& r) {
     if (r.N < 4) return true;
     if (!r.ragged || r.N > 128) return false;
@@ -745,10 +745,10 @@ inline bool one_column_packets(const RowLoad& r) {
 // ones only re-read A per slice: 512,000 rows at N = 512 1.91 -> 2.18 ms).
 // Ragged rows: a slice's edges cut packets and the last slice is partly empty, so
 // only small launches take slices, from 3 whole ones on (us, unsliced / sliced:
-// 10,000 rows of 20 at N = 401 40 / 31, at N = 301 29 / 35; 30,000 of 8 at N = 449 70 /
-// 75; hubs, 120,000 of 13 at N = 510 449 / 423, 60,000 of 24 at N = 301 200 / 244,
-// 200,000 of 12 at N = 401 508 / 590), with hub rows also narrower ones of few nonzeros, bound by
-// the longest chain (20,000 of 6 at N = 301 39 / 28, of 24 62 / 71).
+// 10,000 rows of 20 at N = 401 40 / 31, at N = 301 29 / 34; 30,000 of 8 at N = 449 70 /
+// 76; hubs, 120,000 of 13 at N = 510 449 / 423, 60,000 of 24 at N = 301 202 / 244,
+// 200,000 of 12 at N = 401 514 / 595), with hub rows also narrower ones of few
+// nonzeros, bound by the longest chain (20,000 of 6 at N = 301 40 / 29, of 24 61 / 70).
 inline int column_slice(const RowLoad& r, int64_t unsliced_waves) {
     if (r.ragged) {
         if (r.N <= 256) return 0;

@@ -773,8 +773,9 @@ double item_skew(const ra_tile_plan* p) {
            std::max(p->info.num_blocks, 1);
 }
 
-// Waves of the kernel that the chip holds at once (registers: 8 and 16 rows 51-56,
-// 74 and 109 at 1-2, 4 and 8 columns a lane, 32 rows 56, 72, 98 and 140).
+// Waves of the kernel that the chip holds at once (VGPRs and AGPRs at 1, 2, 4 and 8
+// columns a lane: 8 rows 51, 55, 71, 110; 16 rows 45, 50, 70, 102; 32 rows 56, 72, 96,
+// 140).
 int64_t resident_waves(const ra_tile_plan* p, int cpl) {
     constexpr int kCus = 256;
     if (p->info.rows_per_window == 32) return kCus * (cpl == 1 ? 32 : cpl == 2 ? 28 : cpl == 4 ? 20 : 12);
@@ -785,15 +786,16 @@ int64_t resident_waves(const ra_tile_plan* p, int cpl) {
 // All of them while the four times as many waves still find room: a wave then has
 // a quarter of the steps, but all of an item's prologue (its tables, the first
 // indices and keys) and the sum over LDS.  8-row windows of equal length gain up
-// to twice the resident waves (1,000 windows of 15 steps at N = 128 14.0 -> 9.8 us,
-// 2,000 of 15 18.5 -> 17.3) and lose beyond (2,600 of 7.5 15 -> 18, 4,000 of 25 44 ->
-// 68); 16-row ones up to 0.8 times, 32-row ones 0.6, where they are long 0.9 (N = 128: 500 of 16 steps
-// 16.2 -> 13.4, 500 of 8 8.6 -> 10.5, 750 of 28 20 -> 18; N = 64: 1,000 of 4 5.9 ->
-// 5.1).  The longer the longest item against the mean one, the later that is: its
-// chain would outlast the rest (3,000 8-row windows of 15 steps, the longest 4 times
-// the mean, 33 -> 24 us), until the shared ones alone do as well (5,000 of 15 at N =
-// 128 71 against 81 for all).  Items of fewer than 6 steps (4 tall) do not pay for it
-// (2,000 of 5 at N = 256 17 -> 20).
+// to twice the resident waves (N = 128: 1,000 windows of 15 steps 12.4 -> 9.6 us, 2,000
+// of 15 18.6 -> 18.5) and lose beyond (2,600 of 7.5 15 -> 18, 4,000 of 25 44 -> 68);
+// 16-row ones up to 0.8 times, 32-row ones 0.6, where they are long 0.9 (N = 128: 500
+// of 16 steps 12.2 -> 11.8, 500 of 8 8.7 -> 10.6, 750 of 28 23.3 -> 20.4; N = 64: 1,000
+// of 4 6.2 -> 5.3).  The longer the longest item against the mean one, the later that
+// is: its chain would outlast the rest (3,000 8-row windows of 15 steps at N = 64, the
+// longest 3.3 times the mean, 30 -> 20 us, 23 with the long ones shared), until the
+// shared long ones alone do as well (5,000 of 15 at N = 128 71 against 81 for all).
+// Items of fewer than 6 steps (4 tall) do not pay for it (2,000 of 5 at N = 256 17 ->
+// 20).
 // Otherwise the long ones, where they are exceptional (twice the mean), whose
 // chains of gathers (128 steps of ~0.6 us in a window of 512 blocks) outlast the
 // rest of a small launch: 50,000 rows of 80 at N = 128 91 -> 84 us, 20,000 of 60 at
@@ -840,9 +842,10 @@ bool half_buffer_fits(int64_t K, int64_t ldb) { return (K + 1) * ldb * 2 <= int6
 // Windows of about equal length sweep in step by themselves, which shows as soon
 // as the rows of B they sweep (one slice of them where the slices are outermost)
 // pass the 4 MB of an L2 by some; us, buffer / pointers at N = 256: 28,000 rows of
-// 60 75 / 66, 32,000 of 100 135 / 125; at N = 128: 48,000 of 40 45 / 41; but 32,000 of 60
-// at N = 64 (4 MB) 22 / 23; at N = 32, where short windows and less
-// even ones lose: 128,000 of 60 91 / 73, 144,000 of 12 29 / 34, 96,000 of 60 (6 MB) 57 / 66.  Shared items have no step to keep.
+// 60 75 / 66, 32,000 of 100 135 / 125; at N = 128: 48,000 of 40 46 / 43; but 32,000 of 60
+// at N = 64 (4 MB) 22 / 23; at N = 32, where short windows and less even ones lose:
+// 128,000 of 60 91 / 73, 144,000 of 12 29 / 34, 96,000 of 60 (6 MB) 57 / 66.  Shared
+// items have no step to keep.
 // Unequal ones only where the gathers bound the launch: 100,000 rows of 60 at N =
 // 256 32.5 and 34.8 % L2 hits, 357 and 352 us; 250,000 of 500 at N = 512 8,880 and 8,800;
 // 150,000 of 100 at N = 256 880 and 871.  With fewer bytes (50,000 of 80 at N = 128: 91 and
