@@ -66,12 +66,13 @@ def test_packets_and_slices_of_ragged_rows(oracle, rows, mean, widths):
                             oracle.spmm_f64(g.rowptr, g.colind, np.abs(g.vals), np.abs(B)), 1e-5, f"zo N={N}")
 
 
-@pytest.mark.parametrize("N", [47, 129, 258])
-def test_resumed_chains_at_ragged_widths(oracle, monkeypatch, N):
+# (30, 210,000): 25 MB of B, one column a lane.
+@pytest.mark.parametrize("N,K", [(47, 900), (129, 900), (258, 900), (30, 210_000)])
+def test_resumed_chains_at_ragged_widths(oracle, monkeypatch, N, K):
     """The FP32 route over column partitions continues each element's chain from C: a packet that overlaps its
     neighbour must neither add to the neighbour's columns twice nor store them."""
     monkeypatch.setenv("RA_TILE_COL_PARTS", "4")
-    g = S.random_csr(400, 900, 40.0, seed=N)
+    g = S.random_csr(400, K, 40.0, seed=N)
     B = _B(g.K, N, seed=N)
     rp, ci, vl = g.torch("cuda")
     plan = ra_spmm.make_tc_direct_plan(rp, ci, vl, g.M, g.K, N)
