@@ -796,11 +796,11 @@ int64_t resident_waves(const ra_tile_plan* p, int cpl) {
 // shared long ones alone do as well (5,000 of 15 at N = 128 71 against 81 for all).
 // Items of fewer than 6 steps (4 tall) do not pay for it (2,000 of 5 at N = 256 17 ->
 // 20).
-// Otherwise the long ones, where they are exceptional (twice the mean), whose
-// chains of gathers (128 steps of ~0.6 us in a window of 512 blocks) outlast the
-// rest of a small launch: 50,000 rows of 80 at N = 128 91 -> 84 us, 20,000 of 60 at
-// N = 64 42 -> 21; of 6,000 windows of 200 blocks each all would be long (N = 64 84 ->
-// 102).  Where the gathered bytes take longer than any chain (1.75 GiB, ~200 us)
+// Otherwise the long ones, where they are exceptional (the longest twice the mean,
+// or at most a quarter of the items), whose chains of gathers (128 steps of ~0.6 us
+// in a window of 512 blocks) outlast the rest of a small launch: 50,000 rows of 80
+// at N = 128 91 -> 84 us, 20,000 of 60 at N = 64 42 -> 21; of 6,000 windows of 200
+// blocks each all would be long (N = 64 84 -> 102).  Where the gathered bytes take longer than any chain (1.75 GiB, ~200 us)
 // it only spreads the columns that are gathered at a time: 100,000 rows of 60 at N
 // = 256 33 -> 31 % L2 hits, 371 -> 387 us.
 int shared_items(const ra_tile_plan* p, const Part& part, int N, int nslices, int cpl) {
@@ -811,7 +811,8 @@ int shared_items(const ra_tile_plan* p, const Part& part, int N, int nslices, in
     const double room = tall ? (steps < 6 || p->info.rows_per_window == 16 ? 0.8 : 0.6 + 0.015 * std::max(steps - 8, 0.0)) + more
                              : std::min(2.0 + 1.4 * more, 4.0);
     if (kWavesPerBlock * waves <= room * resident_waves(p, cpl) && steps >= (tall ? 4 : 6)) return part.num_items;
-    return skew >= 2 && gathered_bytes(p, N) < kGatherBound ? part.num_long : 0;
+    const bool exceptional = skew >= 2 || 4 * static_cast<int64_t>(part.num_long) <= part.num_items;
+    return exceptional && gathered_bytes(p, N) < kGatherBound ? part.num_long : 0;
 }
 
 TileLaunch tile_launch(const ra_tile_plan* p, const Part& part, const float* C, const float* scratch, int N,
